@@ -358,4 +358,16 @@ D3S_HD float d3s_uniform(uint64_t seed, uint64_t stream, uint64_t index) {
   return (float)(w >> 8) * 0x1.0p-24f;
 }
 
+/* The four uniforms 4q .. 4q + 3 of draw call `stream` under `seed`: d3s_uniform's,
+ * all four words of one block. */
+D3S_HD void d3s_uniform4(uint64_t seed, uint64_t stream, uint64_t q, float *out) {
+  d3s_u32x4 c;
+  c.v[0] = (uint32_t)q;
+  c.v[1] = (uint32_t)(q >> 32);
+  c.v[2] = (uint32_t)stream;
+  c.v[3] = (uint32_t)(stream >> 32);
+  const d3s_u32x4 o = d3s_philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
+  for (int j = 0; j < 4; j++) out[j] = (float)(o.v[j] >> 8) * 0x1.0p-24f;
+}
+
 #endif /* D3S_MATH_H */
