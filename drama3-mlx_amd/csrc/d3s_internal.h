@@ -102,8 +102,10 @@ void launch_ras_select(const RasArgs &r, const int32_t *first, const int32_t *re
 void *stream_workspace(hipStream_t s, size_t bytes);
 /* Waits for the stream, then frees its block and the blocks it outgrew. */
 int release_stream_workspace(hipStream_t s);
-/* Launch the head's gemv. */
+/* Launch the head's gemv: up to two rows by k_linear, more by launch_linear_rows. */
 void launch_linear(const LinearArgs &la, hipStream_t s);
+/* Launch the gemv of several rows on the matrix cores (the same bits). */
+void launch_linear_rows(const LinearArgs &la, hipStream_t s);
 /* Launch the fused head: the gemv's logits and their sample in one launch
  * (k <= 64, V <= head_max_vocab(), at most head_max_rows() rows).  ws: device memory of
  * ws_bytes (at least head_workspace_bytes) whose first split_counter_bytes()
