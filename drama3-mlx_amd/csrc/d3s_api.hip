@@ -83,6 +83,38 @@ void *stream_workspace(hipStream_t s, size_t bytes) {
   return p;
 }
 
+/* stream_workspace for a route that another kernel can take without one: no
+ * allocation while the stream is being captured, nothing that another
+ * stream's capture forbids (the block is cleared by a kernel on `s`) */
+void *stream_workspace_optional(hipStream_t s, size_t bytes) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+  std::lock_guard<std::mutex> lock(g_ws_mutex);
+  const Key key{dev, (uintptr_t)s};
+  Block &b = g_ws[key];
+  if (b.bytes >= bytes) return b.ptr;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  const size_t want = (bytes + (1u << 20) - 1) & ~(size_t)((1u << 20) - 1); /* whole MiB */
+  void *p = nullptr;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  const hipError_t rc = hipMalloc(&p, want);
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (rc != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  launch_zero_fill((uint32_t *)p, want / 4, s);
+  if (b.ptr) g_retired[key].push_back(b.ptr);
+  b.ptr = p;
+  b.bytes = want;
+  return p;
+}
+
 int release_stream_workspace(hipStream_t s) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return D3S_ERR_LAUNCH;
@@ -151,6 +183,15 @@ size_t routed_workspace_bytes(const d3s::SampleArgs &a, d3s::Dtype dt) {
   return 0;
 }
 
+/* the workspace the selecting kernels would use (after the counters' block),
+ * 0 when they do not take the call.  It is not required: without it the
+ * streaming kernel takes the rows (the same bits). */
+size_t select_workspace_bytes(const d3s::SampleArgs &a, d3s::Dtype dt, bool one_row) {
+  if ((a.flags & D3S_FLAG_GENERIC) != 0u || !d3s::sel_takes(a) || d3s::split_segments(a, dt) > 0) return 0;
+  if (a.k <= 64 && a.vocab <= d3s::wide_max_vocab(dt)) return 0;
+  return d3s::split_counter_bytes() + d3s::sel_workspace_bytes(a, dt, one_row);
+}
+
 /* Where a call's workspace comes from: the block the library keeps for the
  * stream (allocated on the first call that needs one), the allocation-free
  * entry point's static scratch, or the caller's memory. */
@@ -207,6 +248,14 @@ int sample_routed(const d3s::SampleArgs &a, d3s::Dtype dt, hipStream_t s, Ws w) 
     if (!w.ptr || w.bytes < off + d3s::bigk_row_bytes(a)) return w.short_rc;
     if (!d3s::launch_bigk(a, dt, (char *)w.ptr + off, w.bytes - off, s)) return w.short_rc;
     return launched();
+  }
+  if (const size_t need = select_workspace_bytes(a, dt, false)) { /* k up to 4096: the selecting kernels */
+    const size_t off = d3s::split_counter_bytes();
+    if (!w.ptr && w.lazy) {
+      w.ptr = d3s::stream_workspace_optional(s, need);
+      w.bytes = w.ptr ? need : 0; /* without one: the streaming kernel */
+    }
+    if (w.ptr && w.bytes > off && d3s::launch_select(a, dt, (char *)w.ptr + off, w.bytes - off, s)) return launched();
   }
   if (!d3s::launch_generic(a, dt, s)) return D3S_ERR_UNSUPPORTED;
   return launched();
@@ -293,9 +342,15 @@ int sample_call(const void *logits, int dtype, int64_t n_rows, int64_t vocab, in
   if (mode == WsMode::Caller) {
     const int rc = check_caller_ws(ws, ws_bytes, need);
     if (rc != D3S_OK) return rc;
-    return sample_routed(a, dt, s, fixed_ws(need ? ws : nullptr, (size_t)ws_bytes, D3S_ERR_WORKSPACE));
+    /* (a workspace the route does not require is used where it can be) */
+    const bool use = need > 0 || (ws && (uintptr_t)ws % 256u == 0u && select_workspace_bytes(a, dt, true) > 0);
+    return sample_routed(a, dt, s, fixed_ws(use ? ws : nullptr, (size_t)ws_bytes, D3S_ERR_WORKSPACE));
   }
   void *p = nullptr;
+  if (need == 0) {
+    const size_t one = select_workspace_bytes(a, dt, true);
+    if (one > 0 && one <= D3S_SCRATCH_BYTES) p = device_scratch();
+  }
   if (need > 0) { /* the segmented kernel, the sorting kernels one row at a time, or the nucleus
                      ids path's filed rows (more rows than the scratch lists: the full path) */
     if (d3s::split_segments(a, dt) > 0 && need > D3S_SCRATCH_BYTES) return D3S_ERR_SCRATCH;
@@ -576,8 +631,11 @@ int64_t d3s_sample_workspace_bytes(int dtype, int64_t n_rows, int64_t vocab, int
   a.k = k;
   a.n_rows = (int)n_rows;
   a.flags = flags;
+  a.opgraph = d3s::op_graph_order(a.vocab, k, (flags & D3S_FLAG_OP_GRAPH) != 0u);
+  const d3s::Dtype dt = dtype == D3S_DTYPE_F32 ? d3s::DT_F32 : d3s::DT_BF16;
   /* probs and cand absent: the ids-only routes, which need the most */
-  return (int64_t)round256(routed_workspace_bytes(a, dtype == D3S_DTYPE_F32 ? d3s::DT_F32 : d3s::DT_BF16));
+  const size_t need = routed_workspace_bytes(a, dt);
+  return (int64_t)round256(need == 0 && k > 64 ? select_workspace_bytes(a, dt, false) : need);
 }
 
 int d3s_workspace_init(void *workspace, int64_t bytes, void *stream) {

@@ -100,6 +100,9 @@ void launch_ras_select(const RasArgs &r, const int32_t *first, const int32_t *re
  * outgrows is kept (a call on another thread may still be enqueueing on it)
  * until release_stream_workspace.  Null when the allocation fails. */
 void *stream_workspace(hipStream_t s, size_t bytes);
+/* The same for a route that can do without: null while `s` is being captured
+ * (unless the block it has is large enough). */
+void *stream_workspace_optional(hipStream_t s, size_t bytes);
 /* Waits for the stream, then frees its block and the blocks it outgrew. */
 int release_stream_workspace(hipStream_t s);
 /* Launch the head's gemv: up to two rows by k_linear, more by launch_linear_rows. */
@@ -151,6 +154,14 @@ int fused_max_vocab(Dtype dt);
 bool launch_topp(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hipStream_t s);
 int topp_max_vocab();
 size_t topp_workspace_bytes(const SampleArgs &a);
+/* Launch the selecting kernels (op graph's order, k up to 4096, rows longer
+ * than the nucleus kernel takes): each row cut into segments, the elements
+ * that can rank below k gathered in ws and ranked by one workgroup.  Rows go
+ * in launches of as many as ws holds; sel_workspace_bytes is for all of them
+ * (up to 256 MiB) or for one row.  Returns false when the call does not fit. */
+bool launch_select(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hipStream_t s);
+bool sel_takes(const SampleArgs &a);
+size_t sel_workspace_bytes(const SampleArgs &a, Dtype dt, bool one_row);
 /* Launch the streaming generic kernel (any V, k <= generic_max_k()). */
 bool launch_generic(const SampleArgs &a, Dtype dt, hipStream_t s);
 int generic_max_k();

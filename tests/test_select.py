@@ -1,0 +1,151 @@
+"""The selecting kernels (64 < k <= 4096 on rows longer than 8192, and small k
+on rows wider than the segmented kernel's) against the oracle, bit for bit:
+row lengths at segment and chunk edges, row starts off 16 bytes, k at its
+limits, ties across the k-th place, rows the kernels leave to the generic
+procedure, and every workspace mode."""
+import numpy as np
+import pytest
+
+import d3s_workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    import d3s
+    import hiprt
+    d3s.lib()
+    if hiprt.device_count() < 1:
+        pytest.skip("no GPU")
+    return d3s
+
+
+def rows(rng, N, stride, dtype, sigma=3.0):
+    x = (rng.standard_normal((N, stride)) * sigma).astype(np.float32)
+    return x if dtype == "f32" else W.f32_to_bf16_bits(x)
+
+
+def check(gpu, oracle, x, u, T, P, **kw):
+    okw = {a: b for a, b in kw.items() if a in ("banned", "vocab")}
+    exp = oracle.sample(x, u, T, P, **okw)
+    got = gpu.sample(x, u, T, P, **kw)
+    assert got["rc"] == 0
+    assert np.array_equal(got["ids"], exp["ids"])
+    if kw.get("want_probs", True):
+        assert np.array_equal(got["cand"], exp["cand"])
+        assert np.array_equal(got["probs"], exp["probs"], equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("N,V,k,T,P", [
+    (1, 8193, 65, 1.0, 0.95), (3, 8197, 1000, 0.7, 0.9), (2, 16384, 4096, 1.0, 1.0), (5, 20001, 129, 0.6, 0.5),
+    (1, 151936, 4095, 1.0, 0.95), (33, 32771, 200, 1.3, 0.99), (2, 270001, 64, 1.0, 0.9), (1, 700001, 1, 1.0, 0.9)])
+def test_shapes(gpu, oracle, dtype, N, V, k, T, P):
+    rng = np.random.default_rng([N, V, k])
+    check(gpu, oracle, rows(rng, N, V, dtype), oracle.uniform(3, 1, N, k), T, P)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_strided_banned_per_row(gpu, oracle, dtype):
+    rng = np.random.default_rng(5)
+    N, V, k = 9, 12345, 300
+    x = rows(rng, N, V + 7, dtype)
+    T = np.array([0.7, 1.0, 0.0, 1e-4, 2.0 ** -21, 2.0 ** 22, 50.0, 1.0, 0.9], np.float32)
+    P = np.array([0.9, 0.0, 0.5, 1.0, 1.5, 0.95, 0.3, 0.999, 0.7], np.float32)
+    ban = np.array([0, -1, V - 1, V, 17, 5, -1, 12000, 1], np.int32)
+    check(gpu, oracle, x, oracle.uniform(4, 1, N, k), T, P, banned=ban, vocab=V)
+
+
+def test_ties_and_special_rows(gpu, oracle):
+    rng = np.random.default_rng(6)
+    V, k = 30011, 500
+    x = rng.standard_normal((14, V)).astype(np.float32) * 2
+    x[0] = 1.5                                   # all equal: more keys than LDS holds
+    x[1] = np.round(x[1])                        # ties by the thousand
+    x[2] = np.round(x[2] * 8) / 8                # ties across the k-th place
+    x[3, 100:] = -np.inf                         # fewer finite values than k
+    x[4] = -np.inf
+    x[5, 777] = np.nan
+    x[6, 29000] = np.inf
+    x[7] *= 1e30                                 # nearly all elements far below the max
+    x[8] *= 1e-30
+    x[9] = 0.0
+    x[9, ::2] = -0.0
+    x[10] = x[10] * 0.01 + 1e6                   # a large offset: x - m in few steps
+    x[11] = -np.abs(x[11]) - 1e4
+    x[12] = np.sort(x[12])[::-1]                 # the top k in one segment
+    x[13] = 3e38 * np.sign(x[13])
+    check(gpu, oracle, x, oracle.uniform(8, 1, 14, k), 1.0, 0.9)
+    check(gpu, oracle, x, oracle.uniform(8, 2, 14, k), 0.7, 0.5)
+    T = np.full(14, np.inf, np.float32)
+    T[7:] = np.nan
+    check(gpu, oracle, x[:3], oracle.uniform(8, 3, 3, k), T[:3], 0.9)
+    check(gpu, oracle, x[7:9], oracle.uniform(8, 3, 2, k), T[7:9], 0.9)
+
+
+def test_zero_and_one_uniforms(gpu, oracle):
+    rng = np.random.default_rng(7)
+    x = rows(rng, 3, 9000, "f32")
+    u = np.zeros((3, 100), np.float32)
+    u[1] = np.float32(1) - np.float32(2.0 ** -24)
+    u[2, 50:] = 0.25
+    check(gpu, oracle, x, u, 1.0, 0.8)
+
+
+def test_workspace_modes_agree(gpu, oracle):
+    """the query's workspace, one that holds a row at a time, none (the streaming
+    kernel), and the allocation-free entry point: the same bits"""
+    rng = np.random.default_rng(8)
+    N, V, k = 5, 60001, 700
+    x, u = rows(rng, N, V, "bf16"), oracle.uniform(9, 1, N, k)
+    need = gpu.workspace_bytes(gpu.DTYPE_BF16, N, V, k)
+    one = gpu.workspace_bytes(gpu.DTYPE_BF16, 1, V, k)
+    assert 0 < one < need
+    for nbytes in (need, one, 300 << 10):
+        ws = gpu.Workspace(nbytes)
+        check(gpu, oracle, x, u, 0.8, 0.95, workspace=ws)
+        check(gpu, oracle, x, u, 0.8, 0.95, workspace=ws, want_probs=False)
+        ws.free()
+    check(gpu, oracle, x, u, 0.8, 0.95, workspace=(None, 0))
+    check(gpu, oracle, x, u, 0.8, 0.95, noalloc=True)
+    check(gpu, oracle, x, u, 0.8, 0.95, flags=gpu.FLAG_GENERIC)
+
+
+@pytest.mark.parametrize("own_workspace", [True, False])
+def test_captured_and_replayed(gpu, oracle, own_workspace):
+    """d3s_sample_ws (the selecting kernels) and d3s_sample on a stream that has
+    no block yet (nothing is allocated under capture: the streaming kernel),
+    captured and replayed with new inputs between the replays"""
+    import ctypes
+    import hiprt
+    H = hiprt.hip()
+    N, V, k = 3, 20011, 150
+    bx, bu, bids = hiprt.DeviceBuffer(4 * N * V), hiprt.DeviceBuffer(4 * N * k), hiprt.DeviceBuffer(4 * N)
+    s = hiprt.Stream()
+    ws = gpu.Workspace(gpu.workspace_bytes(gpu.DTYPE_F32, N, V, k)) if own_workspace else None
+    hiprt.synchronize()
+    graph, exe = ctypes.c_void_p(), ctypes.c_void_p()
+    hiprt.check(H.hipStreamBeginCapture(s.ptr, 0), "begin capture")
+    rc = gpu.sample_raw(bx.ptr, gpu.DTYPE_F32, N, V, V, bu.ptr, k, 0.8, 0.9, None, bids.ptr, stream=s.ptr,
+                        workspace=ws.arg() if ws else None)
+    hiprt.check(H.hipStreamEndCapture(s.ptr, ctypes.byref(graph)), "end capture")
+    assert rc == 0
+    assert set(hiprt.graph_node_types(graph)) == {"kernel"}
+    hiprt.check(H.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0), "instantiate")
+    try:
+        for rep in range(4):
+            x, u = rows(np.random.default_rng(rep), N, V, "f32"), oracle.uniform(1, rep, N, k)
+            bx.upload(x)
+            bu.upload(u)
+            hiprt.synchronize()
+            hiprt.check(H.hipGraphLaunch(exe, s.ptr), "graph launch")
+            s.synchronize()
+            assert np.array_equal(bids.download((N,), np.int32), oracle.sample(x, u, 0.8, 0.9)["ids"]), rep
+            # an eager call between the replays
+            check(gpu, oracle, x, u, 0.8, 0.9, want_probs=False)
+    finally:
+        H.hipGraphExecDestroy(exe)
+        H.hipGraphDestroy(graph)
+        gpu.lib().d3s_stream_workspace_release(s.ptr)
+        s.destroy()
