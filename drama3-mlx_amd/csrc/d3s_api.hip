@@ -183,13 +183,21 @@ size_t routed_workspace_bytes(const d3s::SampleArgs &a, d3s::Dtype dt) {
   return 0;
 }
 
-/* the workspace the selecting kernels would use (after the counters' block),
- * 0 when they do not take the call.  It is not required: without it the
- * streaming kernel takes the rows (the same bits). */
-size_t select_workspace_bytes(const d3s::SampleArgs &a, d3s::Dtype dt, bool one_row) {
-  if ((a.flags & D3S_FLAG_GENERIC) != 0u || !d3s::sel_takes(a) || d3s::split_segments(a, dt) > 0) return 0;
-  if (a.k <= 64 && a.vocab <= d3s::wide_max_vocab(dt)) return 0;
-  return d3s::split_counter_bytes() + d3s::sel_workspace_bytes(a, dt, one_row);
+/* the workspace with which rows go to the selecting kernels (k up to 4096),
+ * or the sorting kernels gather only the keys they need (after the counters'
+ * block); 0 when neither takes the call.  It is not required: without it the
+ * streaming kernel takes the rows, or the sorting kernels all their keys (the
+ * same bits).  one_row: enough for the rows one after the other. */
+size_t optional_workspace_bytes(const d3s::SampleArgs &a, d3s::Dtype dt, bool one_row) {
+  const size_t off = d3s::split_counter_bytes();
+  if (a.k > d3s::generic_max_k()) {
+    if ((a.flags & D3S_FLAG_GENERIC) == 0u && a.vocab <= d3s::topp_max_vocab()) return 0;
+    return one_row ? 0 : off + d3s::bigk_workspace_bytes(a, dt, BIGK_WS_CAP);
+  }
+  if ((a.flags & D3S_FLAG_GENERIC) != 0u || !a.opgraph || a.vocab <= d3s::topp_max_vocab()) return 0;
+  if (d3s::split_segments(a, dt) > 0 || (a.k <= 64 && a.vocab <= d3s::wide_max_vocab(dt))) return 0;
+  if (d3s::sel_takes(a)) return off + d3s::sel_workspace_bytes(a, dt, one_row);
+  return off + d3s::bigk_workspace_bytes(a, dt, one_row ? 1 : BIGK_WS_CAP);
 }
 
 /* Where a call's workspace comes from: the block the library keeps for the
@@ -237,8 +245,18 @@ int sample_routed(const d3s::SampleArgs &a, d3s::Dtype dt, hipStream_t s, Ws w) 
     }
     if (d3s::launch_topp(a, dt, w.ptr, w.bytes, s)) return launched();
   }
+  const size_t off = d3s::split_counter_bytes();
+  if (const size_t want = optional_workspace_bytes(a, dt, false)) {
+    if (!w.ptr && w.lazy) {
+      w.ptr = d3s::stream_workspace_optional(s, want);
+      w.bytes = w.ptr ? want : 0;
+    }
+    if (a.k <= d3s::generic_max_k() && w.ptr && w.bytes > off &&
+        (d3s::launch_select(a, dt, (char *)w.ptr + off, w.bytes - off, s) ||
+         (a.k > 64 && d3s::launch_bigk(a, dt, (char *)w.ptr + off, w.bytes - off, s))))
+      return launched();
+  }
   if (a.k > d3s::generic_max_k()) { /* the sorting kernels, their keys after the counters' block */
-    const size_t off = d3s::split_counter_bytes();
     if (!w.ptr && w.lazy) {
       const size_t need = routed_workspace_bytes(a, dt);
       w.ptr = d3s::stream_workspace(s, need);
@@ -248,14 +266,6 @@ int sample_routed(const d3s::SampleArgs &a, d3s::Dtype dt, hipStream_t s, Ws w) 
     if (!w.ptr || w.bytes < off + d3s::bigk_row_bytes(a)) return w.short_rc;
     if (!d3s::launch_bigk(a, dt, (char *)w.ptr + off, w.bytes - off, s)) return w.short_rc;
     return launched();
-  }
-  if (const size_t need = select_workspace_bytes(a, dt, false)) { /* k up to 4096: the selecting kernels */
-    const size_t off = d3s::split_counter_bytes();
-    if (!w.ptr && w.lazy) {
-      w.ptr = d3s::stream_workspace_optional(s, need);
-      w.bytes = w.ptr ? need : 0; /* without one: the streaming kernel */
-    }
-    if (w.ptr && w.bytes > off && d3s::launch_select(a, dt, (char *)w.ptr + off, w.bytes - off, s)) return launched();
   }
   if (!d3s::launch_generic(a, dt, s)) return D3S_ERR_UNSUPPORTED;
   return launched();
@@ -343,12 +353,12 @@ int sample_call(const void *logits, int dtype, int64_t n_rows, int64_t vocab, in
     const int rc = check_caller_ws(ws, ws_bytes, need);
     if (rc != D3S_OK) return rc;
     /* (a workspace the route does not require is used where it can be) */
-    const bool use = need > 0 || (ws && (uintptr_t)ws % 256u == 0u && select_workspace_bytes(a, dt, true) > 0);
+    const bool use = need > 0 || (ws && (uintptr_t)ws % 256u == 0u && optional_workspace_bytes(a, dt, true) > 0);
     return sample_routed(a, dt, s, fixed_ws(use ? ws : nullptr, (size_t)ws_bytes, D3S_ERR_WORKSPACE));
   }
   void *p = nullptr;
   if (need == 0) {
-    const size_t one = select_workspace_bytes(a, dt, true);
+    const size_t one = optional_workspace_bytes(a, dt, true);
     if (one > 0 && one <= D3S_SCRATCH_BYTES) p = device_scratch();
   }
   if (need > 0) { /* the segmented kernel, the sorting kernels one row at a time, or the nucleus
@@ -635,7 +645,8 @@ int64_t d3s_sample_workspace_bytes(int dtype, int64_t n_rows, int64_t vocab, int
   const d3s::Dtype dt = dtype == D3S_DTYPE_F32 ? d3s::DT_F32 : d3s::DT_BF16;
   /* probs and cand absent: the ids-only routes, which need the most */
   const size_t need = routed_workspace_bytes(a, dt);
-  return (int64_t)round256(need == 0 && k > 64 ? select_workspace_bytes(a, dt, false) : need);
+  const size_t want = k > 64 ? optional_workspace_bytes(a, dt, false) : 0;
+  return (int64_t)round256(need > want ? need : want);
 }
 
 int d3s_workspace_init(void *workspace, int64_t bytes, void *stream) {

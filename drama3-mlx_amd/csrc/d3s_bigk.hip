@@ -1,11 +1,15 @@
-/* The sorting path: the op graph's sampler for k beyond the generic
- * kernel's LDS sort (k > 16384, on rows longer than the nucleus kernel
- * takes), gfx950 wave64.
+/* The sorting path: the op graph's sampler for k beyond the selecting kernels'
+ * (k > 4096 on rows longer than the nucleus kernel takes; k > 16384 without a
+ * workspace that gathers), gfx950 wave64.
  *
  * The reference's op graph (src/sampling.c:22-49) takes any k up to V: with
  * top-k disabled it argsorts the whole row (:33-35).  Each row is cut into
  * up to 16 segments of whole 1024-key tiles, so a launch of few rows still
- * spreads over the CUs; six launches, 1024 threads a workgroup:
+ * spreads over the CUs; six launches, 1024 threads a workgroup.  With k at most
+ * V / 2 the selecting kernels (d3s_select.hip) come first and leave only the
+ * elements that can rank below k ([16, 151936] fp32, k = 8000: 71 us against
+ * 417 us by the streaming kernel; [1024, 20000] bf16, k = 6000: 173 us against
+ * 400 us); otherwise
  *  k_bk_keys (a workgroup per segment): x = L / T, classification and the
  *     segment's max; the composite keys (ordkey(x), ~index) written to the
  *     workspace in index order, with the segment's digit counts for the first
@@ -33,7 +37,7 @@
  * The same definition as the generic and nucleus kernels, bit for bit.  The
  * workspace holds, per row, two buffers of the row's keys (16 bytes per
  * element), the passes' count tables and the segments' records. */
-#include "d3s_generic.h"
+#include "d3s_select.h"
 
 #pragma clang fp contract(off)
 
@@ -52,12 +56,6 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-/* the sort digit of a composite key in a pass: byte `pass` of ~ordkey(x)
- * (ascending ~ordkey is descending x) */
-__device__ __forceinline__ uint32_t bk_digit(uint64_t key, int pass) {
-  return (uint32_t)((~key) >> (32 + 8 * pass)) & 0xffu;
-}
-
 /* the wave's lanes whose d has the same low `bits` bits as this lane's
  * (among the lanes in `live`), by one ballot per bit */
 template <int BITS>
@@ -71,34 +69,11 @@ __device__ __forceinline__ uint64_t wave_peers(uint32_t d, uint64_t live) {
   return peers;
 }
 
-__device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int l) {
-  return ((uint64_t)readlane_u((uint32_t)(v >> 32), l) << 32) | readlane_u((uint32_t)v, l);
-}
-
-/* sum over the wave of per-lane 64-bit values, exact modulo 2^64 (three
- * 24-bit parts, each summed in 32 bits): a thread's partial sum over a long
- * segment of terms near 2^40 can pass the shared wave sum's 2^45 */
-__device__ __forceinline__ uint64_t bk_wave_sum(uint64_t v) {
-  const uint32_t p0 = wave_sum_u32((uint32_t)(v & 0xffffffu));
-  const uint32_t p1 = wave_sum_u32((uint32_t)((v >> 24) & 0xffffffu));
-  const uint32_t p2 = wave_sum_u32((uint32_t)(v >> 48));
-  return (uint64_t)p0 + ((uint64_t)p1 << 24) + ((uint64_t)p2 << 48);
-}
-
-/* inclusive prefix sum over the wave of per-lane 64-bit values, exact
- * modulo 2^64 (three 24-bit parts) */
-__device__ __forceinline__ uint64_t bk_wave_scan(uint64_t v) {
-  const uint32_t p0 = wave_scan_add_u32((uint32_t)(v & 0xffffffu));
-  const uint32_t p1 = wave_scan_add_u32((uint32_t)((v >> 24) & 0xffffffu));
-  const uint32_t p2 = wave_scan_add_u32((uint32_t)(v >> 48));
-  return (uint64_t)p0 + ((uint64_t)p1 << 24) + ((uint64_t)p2 << 48);
-}
-
 /* block sum of per-thread fixed-point values, exact modulo 2^64 (the
  * oracle's integer sums); opens with a barrier (the scratch may still be
  * being read) */
 __device__ __forceinline__ uint64_t bk_block_sum(uint64_t v, uint32_t *lo, uint32_t *hi) {
-  const uint64_t w = bk_wave_sum(v);
+  const uint64_t w = wave_sum_mod64(v);
   __syncthreads();
   if (lane_id() == 0) {
     lo[threadIdx.x / WAVE] = (uint32_t)w;
@@ -111,80 +86,53 @@ __device__ __forceinline__ uint64_t bk_block_sum(uint64_t v, uint32_t *lo, uint3
   return t;
 }
 
-constexpr int BK_SMAX = 16; /* segments per row (at most) */
 constexpr int BK_B = 8;     /* loads a thread keeps in flight in the streaming loops */
 constexpr int BK_PF = 4;    /* tiles of keys a pass keeps in flight (even) */
 constexpr int BK_WGS = 512; /* workgroups a launch aims at: two per CU */
 
-/* a segment's record: its max and refusal flag (k_bk_keys), its exact sum
- * (the row's first pass); then, for the segment's ranks [s L, s L + L) after the
- * sort, the sums of their terms fix40(d3s_expf(x_r - lse)) and
- * fix40(d3s_expf(x_r - x_0)) (k_bk_sums) and their race's first maximum
- * (k_bk_race); segment 0's record also holds the row's cut and 1 / kept sum
- * (k_bk_cut) */
-struct __align__(16) BkMeta {
-  float max;
-  uint32_t flags;
-  uint64_t sum;
-  uint32_t kor, kand; /* OR and AND of the segment's digit words (k_bk_keys) */
-  uint32_t klow;      /* OR of the low 16 bits of its x (k_bk_keys) */
-  uint64_t psum, ksum;
-  float best;
-  int bestr;
-  int cut;
-  float inv;
+/* n positions cut into the row's segments: whole tiles each */
+struct BkCut {
+  uint32_t sl;  /* positions a segment */
+  float inv_sl; /* 1 / sl, rounded */
 };
+__device__ __forceinline__ BkCut bk_cut_of(uint32_t n, const BkLayout &L) {
+  const uint32_t tiles = (n + BK_T - 1) / BK_T;
+  BkCut c;
+  c.sl = max(1u, (tiles + (uint32_t)L.nseg - 1) / (uint32_t)L.nseg) * BK_T;
+  c.inv_sl = 1.0f / (float)c.sl;
+  return c;
+}
 
-/* a launch's rows in the workspace (the tile sums after the records): the rows' key buffers, their count
- * tables ([row][pass][segment][digit]: filled by the pass before each), the
- * segments' counts of digits 0 and 2 in index order ([row][2][segment][digit]:
- * the first pass's, k_bk_keys'), then their segments' records */
-struct BkLayout {
-  uint64_t *keys; /* [n][2][vstride] */
-  uint32_t *hist; /* [n][4][BK_SMAX][NB] */
-  uint32_t *hidx; /* [n][2][BK_SMAX][NB] */
-  BkMeta *meta;   /* [n][BK_SMAX] */
-  uint64_t *tsum; /* [n][ntiles][2]: each tile's exact prefix and kept-sum terms' sums (k_bk_sums) */
-  int ntiles;     /* tiles of BK_T ranks a row */
-  int64_t vstride;
-  int nseg, tps;  /* segments per row, tiles per segment */
-  int pass0;      /* the first pass launched: 2 when every row's x is known to
-                     have zero low 16 bits (bf16 logits at a scalar T of 1),
-                     else 0 */
-  float inv_sl;   /* 1 / (tps BK_T), rounded */
-};
-
-/* the segment holding position pos: pos / (tps BK_T), from a float
+/* the segment holding position pos: pos / sl, from a float
  * estimate within one of it (pos < 2^26 and the segment length are exact
  * in fp32; the product's relative error is below 2^-23) */
-__device__ __forceinline__ uint32_t bk_seg_of(uint32_t pos, const BkLayout &L) {
-  const uint32_t sl = (uint32_t)(L.tps * BK_T);
-  uint32_t q = (uint32_t)((float)pos * L.inv_sl);
-  q = q * sl > pos ? q - 1u : q;
-  q = (q + 1u) * sl <= pos ? q + 1u : q;
+__device__ __forceinline__ uint32_t bk_seg_of(uint32_t pos, const BkCut &c) {
+  uint32_t q = (uint32_t)((float)pos * c.inv_sl);
+  q = q * c.sl > pos ? q - 1u : q;
+  q = (q + 1u) * c.sl <= pos ? q + 1u : q;
   return q;
 }
 
 /* the row's max and refusal flag from its segments' records (every wave
- * alike: lane s reads segment s, all in one round of loads); with S, also
- * the row's exact sum (the first pass's); with fp, the first radix pass the
- * row runs: 4 when every key's x is the same (no pass reorders anything:
- * the keys stay in index order), 2 when every x has its low 16 bits zero
- * (bf16 logits at T = 1), else 0.  In the second case digits 0 and 1 are
+ * alike: lane s reads segment s, all in one round of loads) and the keys they
+ * hold; with S, also the row's exact sum; with fp, the first radix pass the
+ * row runs: 2 when every x has its low 16 bits zero (bf16 logits at T = 1) or
+ * every x is the same, else 0.  In the first case digits 0 and 1 are
  * 0x0000 or 0xffff by x's sign, which digit 3 holds: keys equal in digits 2
  * and 3 are equal in x, so passes 2 and 3 alone, from index order, give the
- * same stable order as all four.  Skipping two keeps the result in the
- * first buffer. */
-__device__ __forceinline__ void bk_row_max(const BkLayout &L, int row, float &M, uint32_t &F, uint64_t *S = nullptr,
-                                           int *fp = nullptr) {
+ * same stable order as all four; in the second no pass reorders anything.
+ * Skipping two keeps the result in the first buffer. */
+__device__ __forceinline__ void bk_row_max(const BkLayout &L, int row, float &M, uint32_t &F, uint32_t *n_keys = nullptr,
+                                           uint64_t *S = nullptr, int *fp = nullptr) {
   const int lane = lane_id();
   const BkMeta *mt = L.meta + (size_t)row * BK_SMAX;
   float m = -__builtin_inff();
-  uint32_t f = 0u, o = 0u, n = ~0u, lw = 0u;
+  uint32_t f = 0u, o = 0u, n = ~0u, lw = 0u, c = 0u;
   uint64_t sm = 0ull;
   if (lane < L.nseg) {
     m = mt[lane].max;
     f = mt[lane].flags;
+    if (n_keys) c = mt[lane].count;
     if (S) sm = mt[lane].sum;
     if (fp) {
       o = mt[lane].kor;
@@ -194,6 +142,7 @@ __device__ __forceinline__ void bk_row_max(const BkLayout &L, int row, float &M,
   }
   M = wave_max_f(m);
   F = __ballot(f & 1u) ? 1u : 0u;
+  if (n_keys) *n_keys = wave_sum_u32(c);
   if (S) {
     uint64_t t = 0ull;
     for (int s2 = 0; s2 < L.nseg; s2++) t += readlane_u64(sm, s2);
@@ -205,7 +154,7 @@ __device__ __forceinline__ void bk_row_max(const BkLayout &L, int row, float &M,
       ro |= readlane_u(o, s2);
       rn &= readlane_u(n, s2);
     }
-    *fp = ro == rn ? 4 : (__ballot(lw != 0u) == 0ull ? 2 : 0);
+    *fp = ro == rn || __ballot(lw != 0u) == 0ull ? 2 : 0;
   }
 }
 
@@ -221,7 +170,7 @@ __global__ __launch_bounds__(BK_T) void k_bk_keys(SampleArgs a, BkLayout L) {
   const int seg = (int)blockIdx.x, row = (int)blockIdx.y;
   const int tid = (int)threadIdx.x, lane = lane_id(), wid = tid / WAVE;
   const int V = a.vocab;
-  const int lo = seg * L.tps * BK_T, hi = min(V, lo + L.tps * BK_T);
+  const int lo = seg * L.rstride, hi = min(V, lo + L.rstride);
   const RowP rp = row_params(a, row);
   const float T = rp.T;
   const bool t_finite = T < __builtin_inff();
@@ -295,13 +244,13 @@ __global__ __launch_bounds__(BK_T) void k_bk_keys(SampleArgs a, BkLayout L) {
       N &= sh_and[w];
       W |= sh_low[w];
     }
-    BkMeta m;
+    BkMeta m{};
     m.max = M;
     m.flags = F;
-    m.sum = 0ull;
     m.kor = O;
     m.kand = N;
     m.klow = W;
+    m.count = (uint32_t)max(hi - lo, 0);
     L.meta[(size_t)row * BK_SMAX + seg] = m;
   }
 }
@@ -316,29 +265,20 @@ __global__ __launch_bounds__(BK_T) void k_bk_pass(SampleArgs a, BkLayout L, int 
   __shared__ uint32_t sh_lo[BK_NW], sh_hi[BK_NW];
   const int seg = (int)blockIdx.x, row = (int)blockIdx.y;
   const int tid = (int)threadIdx.x, lane = lane_id(), wid = tid / WAVE;
-  const int V = a.vocab;
-  const int lo = seg * L.tps * BK_T, hi = min(V, lo + L.tps * BK_T);
   float M;
-  uint32_t F;
+  uint32_t F, n;
   int fp;
-  bk_row_max(L, row, M, F, nullptr, &fp);
+  bk_row_max(L, row, M, F, &n, nullptr, &fp);
   if ((F & 1u) || M == -__builtin_inff()) return; /* (every workgroup of the row alike) */
   uint64_t *buf = L.keys + (size_t)row * 2 * (size_t)L.vstride;
-  if (pass < fp) { /* a pass the row skips; with no pass to run, the first launched takes the sum */
-    if (fp == 4 && pass == L.pass0) {
-      uint64_t acc = 0ull;
-#pragma unroll 1
-      for (int r0 = lo + tid; r0 < hi; r0 += BK_B * BK_T) {
-        uint64_t kv[BK_B];
-#pragma unroll
-        for (int q = 0; q < BK_B; q++) kv[q] = r0 + q * BK_T < hi ? buf[r0 + q * BK_T] : 0ull;
-#pragma unroll
-        for (int q = 0; q < BK_B; q++)
-          if (r0 + q * BK_T < hi) acc += d3s_fix40_exp(key_x(kv[q]) - M); /* (x <= m) */
-      }
-      const uint64_t S = bk_block_sum(acc, sh_lo, sh_hi);
-      if (tid == 0) L.meta[(size_t)row * BK_SMAX + seg].sum = S;
-    }
+  if (pass < fp) return; /* a pass the row skips */
+  /* the row's first pass reads the segments' regions in index order, the later
+   * ones the n keys cut into segments of whole tiles */
+  const BkCut cut = bk_cut_of(n, L);
+  const int lo = pass == fp ? seg * L.rstride : seg * (int)cut.sl;
+  const int hi = pass == fp ? lo + (int)L.meta[(size_t)row * BK_SMAX + seg].count : min((int)n, lo + (int)cut.sl);
+  if (lo >= hi) {
+    if (pass == fp && !L.summed && tid == 0) L.meta[(size_t)row * BK_SMAX + seg].sum = 0ull;
     return;
   }
   const int e = pass - fp; /* the passes run before this one */
@@ -389,6 +329,7 @@ __global__ __launch_bounds__(BK_T) void k_bk_pass(SampleArgs a, BkLayout L, int 
    * outstanding: the pass is bound by that latency, not by its work) */
   const uint64_t lt = (1ull << lane) - 1ull;
   uint64_t acc = 0ull; /* the row's first pass: the segment's exact sum */
+  const bool sums = pass == fp && !L.summed;
   uint64_t pf[BK_PF];
 #pragma unroll
   for (int q = 0; q < BK_PF; q++) pf[q] = lo + q * BK_T + tid < hi ? src[lo + q * BK_T + tid] : 0ull;
@@ -409,7 +350,7 @@ __global__ __launch_bounds__(BK_T) void k_bk_pass(SampleArgs a, BkLayout L, int 
       const uint64_t peers = wave_peers<8>(d, live);
       const uint32_t below = (uint32_t)__popcll(peers & lt);
       if (valid && below == 0u) wcnt[par][wid][d] = (uint32_t)__popcll(peers);
-      if (pass == fp && valid) acc += d3s_fix40_exp(key_x(key) - M); /* (the row's first pass; x <= m) */
+      if (sums && valid) acc += d3s_fix40_exp(key_x(key) - M); /* (x <= m) */
       lds_barrier();
       if (tid < NB) {
         uint32_t run = base[tid];
@@ -427,7 +368,7 @@ __global__ __launch_bounds__(BK_T) void k_bk_pass(SampleArgs a, BkLayout L, int 
         const uint32_t pos = wcnt[par][wid][d] + below;
         dst[pos] = key;
         if (pass < 3) { /* the segment the key lands in, for the next pass */
-          const uint32_t ds = bk_seg_of(pos, L);
+          const uint32_t ds = bk_seg_of(pos, cut);
           atomicAdd(&nxt[ds * NB + bk_digit(key, pass + 1)], 1u);
         }
       }
@@ -441,7 +382,7 @@ __global__ __launch_bounds__(BK_T) void k_bk_pass(SampleArgs a, BkLayout L, int 
       if (c) atomicAdd(&gn[j], c);
     }
   }
-  if (pass == fp) {
+  if (sums) {
     const uint64_t S = bk_block_sum(acc, sh_lo, sh_hi);
     if (tid == 0) L.meta[(size_t)row * BK_SMAX + seg].sum = S;
   }
@@ -453,14 +394,14 @@ __device__ __forceinline__ bool bk_row_lse(const BkLayout &L, int row, float &ls
   float M;
   uint32_t F;
   uint64_t S;
-  bk_row_max(L, row, M, F, &S);
+  bk_row_max(L, row, M, F, nullptr, &S);
   if ((F & 1u) || M == -__builtin_inff()) return false;
   lse = M + d3s_logf(d3s_fixsum_to_f32(S));
   return true;
 }
 
 /* The op graph's tail (generic_tail_opgraph's definition, bit for bit) over
- * the first k ranks, the ranks cut into the sort's segments:
+ * the first k ranks, cut into segments:
  *  k_bk_sums (a workgroup per segment): the segment's sums of the exact
  *    prefix terms fix40(d3s_expf(x_r - lse)) and of the kept-sum terms
  *    fix40(d3s_expf(x_r - x_0)) (integers: any order);
@@ -477,11 +418,13 @@ __global__ __launch_bounds__(BK_T) void k_bk_sums(SampleArgs a, BkLayout L) {
   const int seg = (int)blockIdx.x, row = (int)blockIdx.y, tid = (int)threadIdx.x;
   const int lane = lane_id(), wid = tid / WAVE;
   float lse;
+  const int k = a.k;
   if (!bk_row_lse(L, row, lse)) return;
   const uint64_t *glist = L.keys + (size_t)row * 2 * (size_t)L.vstride;
   uint64_t *ts = L.tsum + (size_t)row * 2 * (size_t)L.ntiles;
   const float v0 = key_x(glist[0]);
-  const int lo = seg * L.tps * BK_T, hi = min(a.k, lo + L.tps * BK_T);
+  const int SL = (int)bk_cut_of((uint32_t)k, L).sl;
+  const int lo = seg * SL, hi = min(k, lo + SL);
   /* wave w: the segment's tiles w, w + 16, ...; lane l the tile's ranks
    * l + 64 q; each tile's two sums filed, the wave's totals kept */
   uint64_t wp = 0ull, wk = 0ull;
@@ -498,8 +441,8 @@ __global__ __launch_bounds__(BK_T) void k_bk_sums(SampleArgs a, BkLayout L) {
         ps += d3s_fix40_exp(x - lse); /* (x <= x_0 <= lse) */
         ks += d3s_fix40_exp(x - v0);
       }
-    ps = bk_wave_sum(ps);
-    ks = bk_wave_sum(ks);
+    ps = wave_sum_mod64(ps);
+    ks = wave_sum_mod64(ks);
     if (lane == 0) {
       ts[2 * t] = ps;
       ts[2 * t + 1] = ks;
@@ -533,7 +476,7 @@ __global__ __launch_bounds__(BK_T) void k_bk_cut(SampleArgs a, BkLayout L) {
   const uint64_t *glist = L.keys + (size_t)row * 2 * (size_t)L.vstride;
   BkMeta *mt = L.meta + (size_t)row * BK_SMAX;
   const float v0 = key_x(glist[0]);
-  const int SL = L.tps * BK_T;
+  const int SL = (int)bk_cut_of((uint32_t)k, L).sl;
   const int nrs = (k + SL - 1) / SL; /* segments holding ranks below k */
   /* the first segment whose end passes top_p (its prefix before: base);
    * lane s holds segment s's sums */
@@ -569,7 +512,7 @@ __global__ __launch_bounds__(BK_T) void k_bk_cut(SampleArgs a, BkLayout L) {
       for (int t0 = lo / BK_T; t0 < t_hi; t0 += WAVE) {
         const int t = t0 + lane;
         const uint64_t pt = t < t_hi ? ts[2 * t] : 0ull, kt = t < t_hi ? ts[2 * t + 1] : 0ull;
-        const uint64_t pin = bk_wave_scan(pt), kin = bk_wave_scan(kt);
+        const uint64_t pin = wave_scan_mod64(pt), kin = wave_scan_mod64(kt);
         const uint64_t m = __ballot(t < t_hi && d3s_fixsum_to_f32(b + pin) > top_p);
         if (m) {
           const int j = (int)__builtin_ctzll(m);
@@ -620,7 +563,8 @@ __global__ __launch_bounds__(BK_T) void k_bk_race(SampleArgs a, BkLayout L) {
   if (!bk_row_lse(L, row, lse)) return;
   const uint64_t *glist = L.keys + (size_t)row * 2 * (size_t)L.vstride;
   BkMeta *mt = L.meta + (size_t)row * BK_SMAX;
-  const int lo = seg * L.tps * BK_T, hi = min(k, lo + L.tps * BK_T);
+  const int SL = (int)bk_cut_of((uint32_t)k, L).sl;
+  const int lo = seg * SL, hi = min(k, lo + SL);
   if (lo >= hi) return;
   const int cut = mt[0].cut;
   const float inv = mt[0].inv;
@@ -678,10 +622,11 @@ __global__ __launch_bounds__(BK_T) void k_bk_race(SampleArgs a, BkLayout L) {
 __global__ __launch_bounds__(WAVE) void k_bk_pick(SampleArgs a, BkLayout L) {
   const int row = (int)blockIdx.x, lane = lane_id();
   float lse;
+  const int k = a.k;
   if (!bk_row_lse(L, row, lse)) return;
   const BkMeta *mt = L.meta + (size_t)row * BK_SMAX;
-  const int SL = L.tps * BK_T;
-  const int nrs = (a.k + SL - 1) / SL;
+  const int SL = (int)bk_cut_of((uint32_t)k, L).sl;
+  const int nrs = (k + SL - 1) / SL;
   float b = -2.0f;
   int r = 0x7fffffff;
   if (lane < nrs) {
@@ -699,37 +644,53 @@ static int64_t bigk_vstride(int vocab) { return ((int64_t)vocab + 63) & ~(int64_
 
 /* per row: two key buffers, six count tables, the segments' records, the
  * tile sums */
-size_t bigk_row_bytes(const SampleArgs &a) {
-  return 2 * (size_t)bigk_vstride(a.vocab) * sizeof(uint64_t) + 6 * (size_t)BK_SMAX * NB * sizeof(uint32_t) +
-         (size_t)BK_SMAX * sizeof(BkMeta) + 2 * (size_t)((a.vocab + BK_T - 1) / BK_T) * sizeof(uint64_t);
+static size_t row_bytes(int64_t vstride) {
+  return 2 * (size_t)vstride * sizeof(uint64_t) + 6 * (size_t)BK_SMAX * NB * sizeof(uint32_t) +
+         (size_t)BK_SMAX * sizeof(BkMeta) + 2 * (size_t)((vstride + BK_T - 1) / BK_T) * sizeof(uint64_t);
+}
+
+size_t bigk_row_bytes(const SampleArgs &a) { return row_bytes(bigk_vstride(a.vocab)); }
+
+/* The selecting front where it leaves at least half of the elements out (its
+ * three launches against k_bk_keys: about 10 us more at [64, 151936] when
+ * nothing is left out). */
+static bool front_helps(const SampleArgs &a) { return 2 * (int64_t)a.k <= a.vocab; }
+
+static size_t front_row_bytes(const SelLayout &F) { return row_bytes(F.vstride) + sel_front_bytes(F, false); }
+
+size_t bigk_workspace_bytes(const SampleArgs &a, Dtype dt, size_t cap) {
+  size_t row = bigk_row_bytes(a);
+  if (front_helps(a)) {
+    SelLayout F{};
+    sel_front_shape(F, a, dt, a.n_rows);
+    row = front_row_bytes(F);
+  }
+  const size_t all = row * (size_t)a.n_rows;
+  return all <= cap ? all : (cap > row ? cap : row);
 }
 
 bool launch_bigk(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hipStream_t s) {
-  const size_t per_row = bigk_row_bytes(a);
-  if (!ws || ws_bytes < per_row || a.vocab < 1) return false;
-  const int64_t chunk = (int64_t)(ws_bytes / per_row);
-  const int es = dt == DT_F32 ? 4 : 2;
-  const int64_t vstride = bigk_vstride(a.vocab);
-  const int tiles = (a.vocab + BK_T - 1) / BK_T;
+  const size_t plain = bigk_row_bytes(a);
+  if (!ws || ws_bytes < plain || a.vocab < 1) return false;
+  int64_t chunk = (int64_t)(ws_bytes / plain);
+  if (chunk > a.n_rows) chunk = a.n_rows;
+  if (chunk > 32768) chunk = 32768; /* (a grid's second dimension) */
+  /* with the front when its rows fit, half as many a launch at the least */
+  SelLayout F{};
+  bool front = false;
+  if (front_helps(a))
+    for (int64_t c = chunk; c > 0 && !front; c = c > chunk - chunk / 2 ? c - 1 : 0) {
+      sel_front_shape(F, a, dt, c);
+      if (front_row_bytes(F) * (size_t)c <= ws_bytes) {
+        front = true;
+        chunk = c;
+      }
+    }
+  const int64_t vstride = front ? F.vstride : bigk_vstride(a.vocab);
   for (int64_t r0 = 0; r0 < a.n_rows; r0 += chunk) {
-    SampleArgs c = a;
     const int64_t n = a.n_rows - r0 < chunk ? a.n_rows - r0 : chunk;
-    c.n_rows = (int)n;
-    c.logits = (const char *)a.logits + (size_t)r0 * (size_t)a.row_stride * es;
-    c.u = a.u + (size_t)r0 * a.k;
-    if (a.temperature) c.temperature = a.temperature + r0;
-    if (a.top_p) c.top_p = a.top_p + r0;
-    if (a.banned) c.banned = a.banned + r0;
-    c.ids = a.ids + r0;
-    if (a.probs) c.probs = a.probs + (size_t)r0 * a.k;
-    if (a.cand) c.cand = a.cand + (size_t)r0 * a.k;
-    /* segments: enough workgroups for the CUs, whole tiles each */
-    int want = (int)((BK_WGS + n - 1) / n);
-    want = want < 1 ? 1 : (want > BK_SMAX ? BK_SMAX : want);
+    const SampleArgs c = rows_from(a, dt, r0, n);
     BkLayout L{};
-    L.tps = (tiles + want - 1) / want;
-    L.nseg = (tiles + L.tps - 1) / L.tps;
-    L.inv_sl = 1.0f / (float)(L.tps * BK_T);
     /* bf16 logits at T = 1 (after the clamp to 1e-5 either way): x = L, whose
      * low 16 bits are zero, so every row skips passes 0 and 1 (bk_row_max) */
     L.pass0 = dt == DT_BF16 && !a.temperature && a.temperature_scalar == 1.0f ? 2 : 0;
@@ -738,13 +699,31 @@ bool launch_bigk(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hipSt
     L.hist = (uint32_t *)((char *)ws + (size_t)n * 2 * (size_t)vstride * sizeof(uint64_t));
     L.hidx = L.hist + (size_t)n * 4 * BK_SMAX * NB;
     L.meta = (BkMeta *)(L.hidx + (size_t)n * 2 * BK_SMAX * NB);
-    L.ntiles = tiles;
+    L.ntiles = (int)((vstride + BK_T - 1) / BK_T);
     L.tsum = (uint64_t *)(L.meta + (size_t)n * BK_SMAX);
+    if (front) {
+      L.nseg = F.nseg;
+      L.rstride = F.segc * (dt == DT_F32 ? 4 : 8);
+      L.summed = true;
+      F.seg = (SelSeg *)(L.tsum + (size_t)n * 2 * (size_t)L.ntiles);
+      F.cnt = (uint32_t *)(F.seg + (size_t)n * SEL_SMAX);
+      F.group = F.cnt + (size_t)n * F.nseg * SEL_NB;
+      launch_select_front(c, dt, &L, F, s);
+    } else {
+      /* segments: enough workgroups for the CUs, whole tiles each */
+      const int tiles = (a.vocab + BK_T - 1) / BK_T;
+      int want = (int)((BK_WGS + n - 1) / n);
+      want = want < 1 ? 1 : (want > BK_SMAX ? BK_SMAX : want);
+      const int tps = (tiles + want - 1) / want;
+      L.nseg = (tiles + tps - 1) / tps;
+      L.rstride = tps * BK_T;
+      const dim3 grid((unsigned)L.nseg, (unsigned)n);
+      if (dt == DT_F32)
+        hipLaunchKernelGGL(k_bk_keys<false>, grid, dim3(BK_T), 0, s, c, L);
+      else
+        hipLaunchKernelGGL(k_bk_keys<true>, grid, dim3(BK_T), 0, s, c, L);
+    }
     const dim3 grid((unsigned)L.nseg, (unsigned)n);
-    if (dt == DT_F32)
-      hipLaunchKernelGGL(k_bk_keys<false>, grid, dim3(BK_T), 0, s, c, L);
-    else
-      hipLaunchKernelGGL(k_bk_keys<true>, grid, dim3(BK_T), 0, s, c, L);
     for (int pass = L.pass0; pass < 4; pass++) hipLaunchKernelGGL(k_bk_pass, grid, dim3(BK_T), 0, s, c, L, pass);
     hipLaunchKernelGGL(k_bk_sums, grid, dim3(BK_T), 0, s, c, L);
     hipLaunchKernelGGL(k_bk_cut, dim3((unsigned)n), dim3(BK_T), 0, s, c, L);

@@ -172,6 +172,9 @@ int generic_max_k();
  * Returns false when ws does not hold one row. */
 bool launch_bigk(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hipStream_t s);
 size_t bigk_row_bytes(const SampleArgs &a);
+/* the workspace with which every row (or as many as `cap` holds) goes in one
+ * launch, with room for the front that gathers the elements the tail needs */
+size_t bigk_workspace_bytes(const SampleArgs &a, Dtype dt, size_t cap);
 /* w[i] = 0 for i < n_words (w 16-byte aligned), by a kernel */
 void launch_zero_fill(uint32_t *w, size_t n_words, hipStream_t s);
 /* u[i] = d3s_uniform(seed, stream_id, i), i < n */

@@ -17,8 +17,8 @@
  *     by bucket, each key's rank from the larger keys of its own bucket, then
  *     the op graph's tail with lse from the segments' sums.
  * A row with more gathered keys than LDS holds (crowded ties at the k-th
- * element), or whose T is not finite, is sampled by the generic procedure in
- * k_sel_sort's workgroup.  Every result is the oracle's bits.
+ * element) is sampled by the generic procedure in k_sel_sort's workgroup.
+ * The sorting path (d3s_bigk.hip) takes the first three as its front.  Every result is the oracle's bits.
  *
  * Bound: latency (four launches; k_sel_sort is one workgroup's chain).
  * [32, 151936] bf16, k = 1000: 3.6 + 10.5 + 8.1 + 13.1 us against 438 us for
@@ -34,156 +34,56 @@
 namespace d3s {
 namespace {
 
-constexpr int SEL_T = 512; /* threads of a segment's workgroup */
-constexpr int SEL_NW = SEL_T / WAVE;
-constexpr int SEL_U = 4;   /* 16-byte loads a lane keeps in flight */
 constexpr int SEL_CAP = 8192; /* keys k_sel_sort ranks */
-
-/* a wave's run of 16-byte chunks of its segment */
-struct SelRun {
-  const uint4 *src; /* the row's first chunk */
-  int off;          /* elements of it before the row */
-  int c0, c1;       /* the wave's chunks [c0, c1) */
-};
-
-template <bool BF16>
-__device__ __forceinline__ SelRun sel_run(const SampleArgs &a, const SelLayout &L, int row, int seg, int wid) {
-  constexpr int ES = BF16 ? 2 : 4, EPC = 16 / ES;
-  const char *rowp = (const char *)a.logits + (size_t)row * (size_t)a.row_stride * ES;
-  SelRun r;
-  r.off = (int)(((uintptr_t)rowp & 15u) / ES);
-  r.src = (const uint4 *)(rowp - r.off * ES);
-  const int nchunks = (r.off + a.vocab + EPC - 1) / EPC;
-  const int wch = (L.segc + SEL_NW - 1) / SEL_NW;
-  const int end = min(nchunks, (seg + 1) * L.segc);
-  r.c0 = min(end, seg * L.segc + wid * wch);
-  r.c1 = min(end, r.c0 + wch);
-  return r;
-}
-
-/* SEL_U 16-byte loads a lane from chunk `base` of the run on (zeros past it) */
-__device__ __forceinline__ void sel_load(const SelRun &r, int base, uint4 (&q)[SEL_U]) {
-#pragma unroll
-  for (int u = 0; u < SEL_U; u++) {
-    const int c = base + u * WAVE + lane_id();
-    q[u] = c < r.c1 ? r.src[c] : make_uint4(0u, 0u, 0u, 0u);
-  }
-}
-
-/* fn(v, p0, ok) for every chunk of the run, `first` the loads of its first
- * SEL_U rows of chunks (issued by the caller ahead of whatever it waits for):
- * v the EPC logits (-inf outside the row and at the banned index), p0 the
- * first one's position, ok the bits of those within the run and the row.
- * Every lane calls fn. */
-template <bool BF16, class Fn>
-__device__ __forceinline__ void sel_chunks(const SelRun &r, int V, int banned, const uint4 (&first)[SEL_U], Fn &&fn) {
-  constexpr int EPC = BF16 ? 8 : 4;
-  const int lane = lane_id();
-  uint4 q[SEL_U], next[SEL_U];
-#pragma unroll
-  for (int u = 0; u < SEL_U; u++) q[u] = first[u];
-  /* one copy of fn's code: the launch's instruction fetch costs more than the
-   * register moves of a rolled loop */
-#pragma unroll 1
-  for (int base = r.c0; base < r.c1; base += SEL_U * WAVE) {
-    sel_load(r, base + SEL_U * WAVE, next);
-    const int end = min(r.c1, base + SEL_U * WAVE);
-#pragma unroll 1
-    for (int cw = base; cw < end; cw += WAVE) { /* cw uniform: the 64 chunks' first */
-      const int p0 = (cw + lane) * EPC - r.off, f0 = cw * EPC - r.off;
-      const uint32_t w[4] = {q[0].x, q[0].y, q[0].z, q[0].w};
-      float v[EPC];
-#pragma unroll
-      for (int e = 0; e < EPC; e++)
-        v[e] = BF16 ? d3s_u2f((e & 1) ? (w[e / 2] & 0xffff0000u) : (w[e / 2] << 16)) : d3s_u2f(w[e]);
-      uint32_t ok = (1u << EPC) - 1u;
-      if (f0 < 0 || f0 + WAVE * EPC > V || cw + WAVE > r.c1 || (unsigned)(banned - f0) < (unsigned)(WAVE * EPC)) {
-        ok = 0u;
-#pragma unroll
-        for (int e = 0; e < EPC; e++) {
-          const bool in = cw + lane < r.c1 && (unsigned)(p0 + e) < (unsigned)V;
-          ok |= (in ? 1u : 0u) << e;
-          if (!in || p0 + e == banned) v[e] = -__builtin_inff();
-        }
-      }
-      fn(v, p0, ok);
-#pragma unroll
-      for (int u = 0; u + 1 < SEL_U; u++) q[u] = q[u + 1];
-    }
-#pragma unroll
-    for (int u = 0; u < SEL_U; u++) q[u] = next[u];
-  }
-}
-
-/* x[e] = v[e] / T for a chunk: the fused division without its range test
- * where every lane's logits allow it (zero divides exactly either way) */
-template <int EPC>
-__device__ __forceinline__ void sel_scale(const float (&v)[EPC], float T, float y, bool t_easy, float (&x)[EPC]) {
-  bool ok = t_easy;
-#pragma unroll
-  for (int e = 0; e < EPC; e++) {
-    const uint32_t ea = (d3s_f2u(v[e]) >> 23) & 0xffu;
-    ok = ok && (ea - 67u <= 160u || v[e] == 0.0f);
-  }
-  if (__all(ok)) {
-#pragma unroll
-    for (int e = 0; e < EPC; e++) {
-      const float q = v[e] * y;
-      const float r = __builtin_fmaf(-q, T, v[e]);
-      x[e] = __builtin_fmaf(r, y, q);
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < EPC; e++) x[e] = d3s_div_rn(v[e], T, y);
-  }
-}
-
-/* what a row's segments' maxima say (every wave alike: lane s reads segment
- * s's): m = max x; false for a row with nothing to gather (refused, all -inf,
- * or T not finite: left to the last kernel) */
-__device__ __forceinline__ bool sel_row_max(const SelLayout &L, int row, float T, float &Lmax, float &M) {
-  const int lane = lane_id();
-  Lmax = wave_maximum_f(lane < L.nseg ? L.seg[(size_t)row * SEL_SMAX + lane].lmax : -__builtin_inff());
-  M = 0.0f;
-  if (!(T < __builtin_inff()) || d3s_isnan(Lmax) || fabsf(Lmax) == __builtin_inff()) return false;
-  M = scale_logit(Lmax, T, 1.0f / T, true);
-  return fabsf(M) < __builtin_inff();
-}
-
-__device__ __forceinline__ bool sel_t_easy(float T) {
-  return ((d3s_f2u(T) >> 23) & 0xffu) - 107u <= 40u; /* d3s_div_rn's range of T */
-}
-
-/* the bucket of z = x - m <= 0 (-inf: the last) */
-__device__ __forceinline__ int sel_bucket(float z) { return (int)fminf(z * -SEL_SCALE, (float)(SEL_NB - 1)); }
 
 template <bool BF16>
 __global__ __launch_bounds__(SEL_T) void k_sel_max(SampleArgs a, SelLayout L) {
   __shared__ float sh[SEL_NW];
+  __shared__ uint32_t shn[SEL_NW];
   const int seg = (int)blockIdx.x, row = (int)blockIdx.y;
   const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
   const SelRun run = sel_run<BF16>(a, L, row, seg, wid);
   uint4 first[SEL_U];
   sel_load(run, run.c0, first);
   const int banned = a.banned ? a.banned[row] : -1;
-  float m = -__builtin_inff();
-  sel_chunks<BF16>(run, a.vocab, banned, first, [&](const auto &v, int, uint32_t) {
+  const float ninf = -__builtin_inff();
+  const float T = a.temperature ? a.temperature[row] : a.temperature_scalar;
+  const bool flat = !(T < __builtin_inff()); /* (only T = +inf asks whether some logit is -inf) */
+  float m = ninf;
+  uint32_t masked = 0u;
+  sel_chunks<BF16>(run, a.vocab, banned, first, [&](const auto &v, int, uint32_t ok) {
+    constexpr int EPC = BF16 ? 8 : 4;
 #pragma unroll
-    for (float f : v) m = fmaximum(m, f);
+    for (int e = 0; e < EPC; e++) m = fmaximum(m, v[e]);
+    if (flat) {
+#pragma unroll
+      for (int e = 0; e < EPC; e++) masked |= v[e] == ninf ? (ok >> e) & 1u : 0u;
+    }
   });
   m = wave_maximum_f(m);
-  if (lane_id() == 0) sh[wid] = m;
+  masked = __ballot(masked != 0u) ? 1u : 0u;
+  if (lane_id() == 0) {
+    sh[wid] = m;
+    shn[wid] = masked;
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int w = 1; w < SEL_NW; w++) m = fmaximum(m, sh[w]);
-    L.seg[(size_t)row * SEL_SMAX + seg].lmax = m;
+    for (int w = 1; w < SEL_NW; w++) {
+      m = fmaximum(m, sh[w]);
+      masked |= shn[w];
+    }
+    SelSeg &sg = L.seg[(size_t)row * SEL_SMAX + seg];
+    sg.lmax = m;
+    sg.masked = masked;
   }
 }
 
-template <bool BF16>
+/* SUMS: each bucket's exact sum as well (for the wide nucleus path) */
+template <bool BF16, bool SUMS>
 __global__ __launch_bounds__(SEL_T) void k_sel_hist(SampleArgs a, SelLayout L) {
   __shared__ __align__(16) uint32_t cnt[SEL_NB];
+  __shared__ __align__(16) uint64_t bsum[SUMS ? SEL_NB : 2];
   __shared__ uint64_t sum[SEL_NW];
   constexpr int PER = SEL_NB / SEL_T;
   static_assert(PER == 4 && SEL_G % PER == 0, "a thread's buckets are 16 bytes of one group");
@@ -195,8 +95,12 @@ __global__ __launch_bounds__(SEL_T) void k_sel_hist(SampleArgs a, SelLayout L) {
   const RowP rp = row_params(a, row);
   const float T = rp.T, y = 1.0f / T;
   ((uint4 *)cnt)[tid] = make_uint4(0u, 0u, 0u, 0u);
-  float Lmax, M;
-  if (!sel_row_max(L, row, T, Lmax, M)) return;
+  if (SUMS) {
+    ((uint4 *)bsum)[2 * tid] = make_uint4(0u, 0u, 0u, 0u);
+    ((uint4 *)bsum)[2 * tid + 1] = make_uint4(0u, 0u, 0u, 0u);
+  }
+  float M;
+  if (sel_row_max(L, row, T, M) != SEL_LIVE) return;
   __syncthreads();
   const bool te = sel_t_easy(T);
   uint64_t acc = 0ull;
@@ -208,15 +112,28 @@ __global__ __launch_bounds__(SEL_T) void k_sel_hist(SampleArgs a, SelLayout L) {
     for (int e = 0; e < EPC; e++) {
       const float z = x[e] - M;
       if ((ok >> e) & 1u) {
-        atomicAdd(&cnt[sel_bucket(z)], 1u);
-        acc += d3s_fix40_exp(z);
+        const int b = sel_bucket(z);
+        const uint64_t f = d3s_fix40_exp(z);
+        atomicAdd(&cnt[b], 1u);
+        if (SUMS)
+          atomicAdd((unsigned long long *)&bsum[b], (unsigned long long)f);
+        else
+          acc += f;
       }
     }
   });
+  const size_t at = (size_t)row * L.nseg + seg;
+  if (SUMS) {
+    __syncthreads();
+    const ulonglong2 p = ((const ulonglong2 *)bsum)[2 * tid], q = ((const ulonglong2 *)bsum)[2 * tid + 1];
+    ulonglong2 *out = (ulonglong2 *)(L.csum + at * SEL_NB);
+    out[2 * tid] = p;
+    out[2 * tid + 1] = q;
+    acc = p.x + p.y + q.x + q.y;
+  }
   acc = wave_sum_mod64(acc);
   if (lane_id() == 0) sum[wid] = acc;
   __syncthreads();
-  const size_t at = (size_t)row * L.nseg + seg;
   const uint4 c = ((const uint4 *)cnt)[tid];
   ((uint4 *)(L.cnt + at * SEL_NB))[tid] = c;
   uint32_t g = c.x + c.y + c.z + c.w;
@@ -231,11 +148,14 @@ __global__ __launch_bounds__(SEL_T) void k_sel_hist(SampleArgs a, SelLayout L) {
   }
 }
 
-template <bool BF16>
-__global__ __launch_bounds__(SEL_T) void k_sel_gather(SampleArgs a, SelLayout L) {
+/* SORT: the sorting path's front (B): composite keys with their digits' counts */
+template <bool BF16, bool SORT>
+__global__ __launch_bounds__(SEL_T) void k_sel_gather(SampleArgs a, SelLayout L, BkLayout B) {
   __shared__ uint32_t part[SEL_NW][SEL_NG], fine[SEL_G], wn[SEL_NW];
+  __shared__ uint32_t dig[SORT ? 2 : 1][NB], wor[SEL_NW], wand[SEL_NW], wlow[SEL_NW];
   static_assert(SEL_NG == WAVE && SEL_SMAX % SEL_NW == 0, "a lane a group");
-  constexpr int EPC = BF16 ? 8 : 4, GL = SEL_SMAX / SEL_NW, FL = SEL_SMAX * SEL_G / SEL_T;
+  constexpr int EPC = BF16 ? 8 : 4, SM = SORT ? BK_SMAX : SEL_SMAX;
+  constexpr int GL = SM / SEL_NW, FL = (SM * SEL_G + SEL_T - 1) / SEL_T;
   const int seg = (int)blockIdx.x, row = (int)blockIdx.y, tid = (int)threadIdx.x;
   const int wid = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int lane = lane_id();
@@ -251,9 +171,27 @@ __global__ __launch_bounds__(SEL_T) void k_sel_gather(SampleArgs a, SelLayout L)
     g[q] = s < L.nseg ? L.group[(at0 + s) * SEL_NG + lane] : 0u;
   }
   const RowP rp = row_params(a, row);
-  const float T = rp.T;
-  float Lmax, M;
-  if (!sel_row_max(L, row, T, Lmax, M)) return;
+  const float T = rp.T, y = 1.0f / T;
+  float M;
+  const SelRow what = sel_row_max(L, row, T, M);
+  uint32_t *hx = nullptr, *gh = nullptr;
+  if (SORT) { /* the passes' counts: this segment's of digits 0 and 2 below; the later ones are added to */
+    gh = B.hist + (size_t)row * 4 * BK_SMAX * NB;
+    hx = B.hidx + (size_t)row * 2 * BK_SMAX * NB;
+    if (tid < NB) {
+      dig[0][tid] = 0u;
+      dig[SORT ? 1 : 0][tid] = 0u;
+#pragma unroll
+      for (int p = 1; p < 4; p++) gh[(p * BK_SMAX + seg) * NB + tid] = 0u;
+    }
+    if (what != SEL_LIVE && tid == 0) {
+      BkMeta m{};
+      m.max = what == SEL_MASKED ? -__builtin_inff() : 0.0f;
+      m.flags = what == SEL_REFUSED ? 1u : 0u;
+      B.meta[(size_t)row * BK_SMAX + seg] = m;
+    }
+  }
+  if (what != SEL_LIVE) return;
   const uint32_t k = (uint32_t)a.k;
 #pragma unroll
   for (int q = 1; q < GL; q++) g[0] += g[q];
@@ -271,7 +209,8 @@ __global__ __launch_bounds__(SEL_T) void k_sel_gather(SampleArgs a, SelLayout L)
 #pragma unroll
   for (int q = 0; q < FL; q++) {
     const int s = tid / SEL_G + q * (SEL_T / SEL_G);
-    f += s < L.nseg ? L.cnt[(at0 + s) * SEL_NB + tg * SEL_G + tid % SEL_G] : 0u;
+    const size_t at = (at0 + s) * SEL_NB + tg * SEL_G + tid % SEL_G;
+    f += s < L.nseg ? L.cnt[at] : 0u;
   }
   if (f) atomicAdd(&fine[tid % SEL_G], f);
   __syncthreads();
@@ -280,9 +219,9 @@ __global__ __launch_bounds__(SEL_T) void k_sel_gather(SampleArgs a, SelLayout L)
   /* every logit of the buckets up to tb reaches Lc: (tb + 1) / SEL_SCALE below
    * m, with room for the roundings of x, of x - m and of this bound (a few
    * elements below them may as well: the set holds every element above any of
-   * its own, which is all that k_sel_sort asks) */
+   * its own, which is all that the ranking asks) */
   float Lc = -__builtin_inff();
-  if (tb < SEL_NB - 1) {
+  if (tb < SEL_NB - 1 && T < __builtin_inff()) {
     const float xc = M - ((float)(tb + 1) * (1.0f / SEL_SCALE)) * 1.0001f;
     Lc = (xc - (fabsf(M) + fabsf(xc) + 1.0f) * 0x1p-20f) * T;
     Lc = Lc - fabsf(Lc) * 0x1p-20f;
@@ -306,20 +245,75 @@ __global__ __launch_bounds__(SEL_T) void k_sel_gather(SampleArgs a, SelLayout L)
     at += w < wid ? wn[w] : 0u;
     tot += wn[w];
   }
-  if (tid == 0) L.seg[(size_t)row * SEL_SMAX + seg].count = tot;
-  if (n == 0u) return;
-  uint64_t *out = L.keys + (size_t)row * (size_t)L.vstride + (size_t)seg * L.segc * EPC;
+  if (!SORT) {
+    if (tid == 0) L.seg[(size_t)row * SEL_SMAX + seg].count = tot;
+    if (n == 0u) return;
+  }
+  uint64_t *out = SORT ? B.keys + (size_t)row * 2 * (size_t)B.vstride + (size_t)seg * B.rstride
+                       : L.keys + (size_t)row * (size_t)L.vstride + (size_t)seg * L.segc * EPC;
+  const bool te = sel_t_easy(T);
+  uint32_t wo = 0u, wa = ~0u, wl = 0u;
   sel_chunks<BF16>(run, a.vocab, rp.banned, first, [&](const auto &v, int p0, uint32_t ok) {
     const uint32_t m = pick(v, ok);
     if (__ballot(m != 0u) == 0ull) return;
     const uint32_t c = (uint32_t)__popc(m);
     const uint32_t inc = wave_scan_add_u32(c);
     uint32_t slot = at + inc - c;
+    if (SORT) {
+      float x[EPC];
+      sel_scale(v, T, y, te, x);
 #pragma unroll
-    for (int e = 0; e < EPC; e++)
-      if ((m >> e) & 1u) out[slot++] = ((uint64_t)d3s_f2u(v[e]) << 32) | (uint32_t)(p0 + e);
+      for (int e = 0; e < EPC; e++)
+        if ((m >> e) & 1u) {
+          const uint64_t key = composite_key(x[e], p0 + e);
+          out[slot++] = key;
+          /* (with pass 0 not launched its counts are not read; its digit is
+           * then one of two values by the sign: 1024 atomics on two words) */
+          if (B.pass0 == 0) atomicAdd(&dig[0][bk_digit(key, 0)], 1u);
+          atomicAdd(&dig[SORT ? 1 : 0][bk_digit(key, 2)], 1u);
+          const uint32_t dw = (uint32_t)((~key) >> 32); /* the digit word */
+          wo |= dw;
+          wa &= dw;
+          wl |= d3s_f2u(x[e]) & 0xffffu;
+        }
+    } else {
+#pragma unroll
+      for (int e = 0; e < EPC; e++)
+        if ((m >> e) & 1u) out[slot++] = ((uint64_t)d3s_f2u(v[e]) << 32) | (uint32_t)(p0 + e);
+    }
     at += readlane_u(inc, 63);
   });
+  if (!SORT) return;
+#pragma unroll
+  for (int sh = 1; sh < WAVE; sh <<= 1) {
+    wo |= (uint32_t)__shfl_xor((int)wo, sh);
+    wa &= (uint32_t)__shfl_xor((int)wa, sh);
+    wl |= (uint32_t)__shfl_xor((int)wl, sh);
+  }
+  if (lane == 0) {
+    wor[wid] = wo;
+    wand[wid] = wa;
+    wlow[wid] = wl;
+  }
+  __syncthreads();
+  if (tid < NB) {
+    hx[seg * NB + tid] = dig[0][tid];
+    hx[(BK_SMAX + seg) * NB + tid] = dig[SORT ? 1 : 0][tid];
+  }
+  if (tid == 0) {
+    BkMeta m{};
+    m.max = M;
+    m.sum = L.seg[(size_t)row * SEL_SMAX + seg].sum;
+    m.kand = ~0u;
+#pragma unroll
+    for (int w = 0; w < SEL_NW; w++) {
+      m.kor |= wor[w];
+      m.kand &= wand[w];
+      m.klow |= wlow[w];
+    }
+    m.count = tot;
+    B.meta[(size_t)row * BK_SMAX + seg] = m;
+  }
 }
 
 /* the op graph's tail (generic_tail_opgraph's definition) over k <= NQ GBLOCK
@@ -426,18 +420,16 @@ __global__ __launch_bounds__(GBLOCK) void k_sel_sort(SampleArgs a, SelLayout L, 
   }
   const RowP rp = row_params(a, row);
   const float T = rp.T, y = 1.0f / T;
-  float Lmax, M;
-  const bool live = sel_row_max(L, row, T, Lmax, M);
-  const uint32_t inc = wave_scan_add_u32(segn);
-  const uint32_t n = live ? readlane_u(inc, WAVE - 1) : 0u;
-  /* T not finite, or a crowded last bucket */
-  const bool generic = live ? n > (uint32_t)SEL_CAP : !(T < __builtin_inff());
-  if (generic) {
-    generic_row<BF16>(a, row, kpow, dyn);
+  float M;
+  const SelRow what = sel_row_max(L, row, T, M);
+  if (what != SEL_LIVE) { /* a NaN or +inf x: refused; every x -inf: masked */
+    write_special(a, row, what == SEL_MASKED);
     return;
   }
-  if (!live) { /* a NaN or +inf x: refused; every x -inf: masked */
-    write_special(a, row, Lmax == -__builtin_inff() || M == -__builtin_inff());
+  const uint32_t inc = wave_scan_add_u32(segn);
+  const uint32_t n = readlane_u(inc, WAVE - 1);
+  if (n > (uint32_t)SEL_CAP) { /* a crowded last bucket */
+    generic_row<BF16>(a, row, kpow, dyn);
     return;
   }
   const float lse = M + d3s_logf(d3s_fixsum_to_f32(wave_sum_mod64(segs)));
@@ -464,7 +456,7 @@ __global__ __launch_bounds__(GBLOCK) void k_sel_sort(SampleArgs a, SelLayout L, 
 #pragma unroll
   for (int q = 0; q < NK; q++)
     if (tid + q * GBLOCK < n) {
-      const float x = scale_logit(d3s_u2f((uint32_t)(kv[q] >> 32)), T, y, true);
+      const float x = scale_logit(d3s_u2f((uint32_t)(kv[q] >> 32)), T, y, T < __builtin_inff());
       kv[q] = composite_key(x, (int)(uint32_t)kv[q]);
       atomicAdd(&next[sel_bucket(x - M)], 1u);
     }
@@ -517,8 +509,8 @@ template <bool BF16>
 void select_rows(const SampleArgs &c, const SelLayout &L, hipStream_t s) {
   const dim3 grid((unsigned)L.nseg, (unsigned)c.n_rows);
   hipLaunchKernelGGL(k_sel_max<BF16>, grid, dim3(SEL_T), 0, s, c, L);
-  hipLaunchKernelGGL(k_sel_hist<BF16>, grid, dim3(SEL_T), 0, s, c, L);
-  hipLaunchKernelGGL(k_sel_gather<BF16>, grid, dim3(SEL_T), 0, s, c, L);
+  hipLaunchKernelGGL((k_sel_hist<BF16, false>), grid, dim3(SEL_T), 0, s, c, L);
+  hipLaunchKernelGGL((k_sel_gather<BF16, false>), grid, dim3(SEL_T), 0, s, c, L, BkLayout{});
   if (c.k <= GBLOCK)
     sort_rows<BF16, 1>(c, L, s);
   else
@@ -530,14 +522,14 @@ int64_t sel_nchunks(const SampleArgs &a, int epc) { return ((int64_t)a.vocab + 2
 
 /* The segments of a row: whole rounds of a workgroup's lanes (SEL_T chunks),
  * as many a segment as leave about SEL_WGS workgroups a launch and at most
- * SEL_SMAX segments a row. */
-void sel_segments(SelLayout &L, const SampleArgs &a, Dtype dt, int64_t rows) {
+ * smax segments a row. */
+void sel_segments(SelLayout &L, const SampleArgs &a, Dtype dt, int64_t rows, int smax) {
   const int epc = dt == DT_F32 ? 4 : 8;
   const int64_t rounds = (sel_nchunks(a, epc) + SEL_T - 1) / SEL_T; /* a row's */
   int64_t want = (SEL_WGS + rows - 1) / rows;
-  if (want > SEL_SMAX) want = SEL_SMAX;
+  if (want > smax) want = smax;
   int64_t per = rounds / want;
-  const int64_t least = (rounds + SEL_SMAX - 1) / SEL_SMAX;
+  const int64_t least = (rounds + smax - 1) / smax;
   if (per < least) per = least;
   L.segc = (int)(per * SEL_T);
   L.nseg = (int)((rounds + per - 1) / per);
@@ -557,7 +549,7 @@ bool sel_takes(const SampleArgs &a) { return a.opgraph && a.k <= SEL_MAX_K && a.
 
 size_t sel_workspace_bytes(const SampleArgs &a, Dtype dt, bool one_row) {
   SelLayout L{};
-  sel_segments(L, a, dt, one_row ? 1 : a.n_rows);
+  sel_segments(L, a, dt, one_row ? 1 : a.n_rows, SEL_SMAX);
   const size_t row = sel_row_bytes(a, L.nseg);
   if (one_row) return row;
   size_t all = row * (size_t)a.n_rows;
@@ -572,7 +564,7 @@ bool launch_select(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hip
   int64_t chunk = a.n_rows < 32768 ? a.n_rows : 32768; /* (a grid's second dimension) */
   SelLayout L{};
   for (;; chunk = (chunk + 1) / 2) {
-    sel_segments(L, a, dt, chunk);
+    sel_segments(L, a, dt, chunk, SEL_SMAX);
     if (sel_row_bytes(a, L.nseg) * (size_t)chunk <= ws_bytes) break;
     if (chunk == 1) return false;
   }
@@ -589,6 +581,35 @@ bool launch_select(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hip
       select_rows<true>(c, L, s);
   }
   return true;
+}
+
+void sel_front_shape(SelLayout &F, const SampleArgs &a, Dtype dt, int64_t rows) {
+  sel_segments(F, a, dt, rows, BK_SMAX);
+}
+
+size_t sel_front_bytes(const SelLayout &F, bool sums) {
+  return (size_t)F.nseg * (sums ? SEL_NB * 12u : (SEL_NB + SEL_NG) * 4u) + SEL_SMAX * sizeof(SelSeg);
+}
+
+namespace {
+template <bool BF16>
+void front(const SampleArgs &a, const BkLayout *L, const SelLayout &F, hipStream_t s) {
+  const dim3 grid((unsigned)F.nseg, (unsigned)a.n_rows);
+  hipLaunchKernelGGL(k_sel_max<BF16>, grid, dim3(SEL_T), 0, s, a, F);
+  if (!L) {
+    hipLaunchKernelGGL((k_sel_hist<BF16, true>), grid, dim3(SEL_T), 0, s, a, F);
+    return;
+  }
+  hipLaunchKernelGGL((k_sel_hist<BF16, false>), grid, dim3(SEL_T), 0, s, a, F);
+  hipLaunchKernelGGL((k_sel_gather<BF16, true>), grid, dim3(SEL_T), 0, s, a, F, *L);
+}
+}  // namespace
+
+void launch_select_front(const SampleArgs &a, Dtype dt, const BkLayout *L, const SelLayout &F, hipStream_t s) {
+  if (dt == DT_F32)
+    front<false>(a, L, F, s);
+  else
+    front<true>(a, L, F, s);
 }
 
 }  // namespace d3s

@@ -149,3 +149,73 @@ def test_captured_and_replayed(gpu, oracle, own_workspace):
         H.hipGraphDestroy(graph)
         gpu.lib().d3s_stream_workspace_release(s.ptr)
         s.destroy()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("sigma", [0.1, 1.0, 3.0, 8.0])
+def test_ids_only_large_k_gathers_the_kept_ranks(gpu, oracle, dtype, sigma):
+    """k > 4096, ids only (the sorting kernels take the ranks top-p can keep):
+    every top_p from 0 to beyond 1, temperatures, banned indices, strides"""
+    rng = np.random.default_rng([int(sigma * 10), dtype == "f32"])
+    V = 24007
+    P = np.array([0.0, 0.1, 0.5, 0.9, 0.95, 0.99, 0.9999, 1.0, 1.5, -1.0, np.nan], np.float32)
+    N = len(P)
+    x = rows(rng, N, V + 3, dtype, sigma)
+    ban = np.where(rng.random(N) < 0.5, rng.integers(0, V, N), -1).astype(np.int32)
+    for T, k in ((1.0, V), (0.7, 17000), (np.linspace(0.3, 2.0, N).astype(np.float32), V), (1.3, 5000)):
+        check(gpu, oracle, x, oracle.uniform(11, 1, N, k), T, P, banned=ban, vocab=V, want_probs=False)
+
+
+def test_ids_only_large_k_special_rows(gpu, oracle):
+    rng = np.random.default_rng(12)
+    V = 20480
+    x = (rng.standard_normal((12, V)) * 3).astype(np.float32)
+    x[0] = 2.0
+    x[1] = np.round(x[1])
+    x[2, 10:] = -np.inf
+    x[3] = -np.inf
+    x[4, 5] = np.nan
+    x[5, V - 1] = np.inf
+    x[6] = x[6] * 0.01 + 1e7      # lse rounds in whole units: no bound on the cut
+    x[7] *= 1e30
+    x[8, 7] = 60.0                # one element holds all the mass
+    x[9] = np.sort(x[9])
+    x[10, ::2] = -0.0
+    x[10, 1::2] = 0.0
+    x[11, 1000:] = -1e30
+    u = oracle.uniform(13, 1, 12, V)
+    for T in (1.0, 0.7, np.inf):
+        check(gpu, oracle, x, u, T, 0.9, want_probs=False)
+    check(gpu, oracle, x, u[:, :6000], 0.9, 0.95, want_probs=False)
+    check(gpu, oracle, x, u[:, :6000], 0.9, 0.95)
+    # kept ranks that cannot win: a dropped rank far past them does
+    u = u.copy()
+    u[:, :15000] = 0.0
+    check(gpu, oracle, x, u, 1.0, 0.9, want_probs=False)
+    u[:, :] = 0.0
+    check(gpu, oracle, x, u, 1.0, 0.9, want_probs=False)
+    u[:, 3:] = 1.0
+    check(gpu, oracle, x, u, 1.0, 0.2, want_probs=False)
+    u[:] = 2.0
+    u[:, 20000] = 0.5
+    check(gpu, oracle, x, u, 1.0, 0.2, want_probs=False)
+
+
+def test_sorting_workspace_modes_agree(gpu, oracle):
+    """the query's workspace, one that holds only the plain sort's keys (what
+    the call requires), and the allocation-free entry point"""
+    rng = np.random.default_rng(14)
+    N, V = 3, 40009
+    x, u = rows(rng, N, V, "bf16"), oracle.uniform(9, 1, N, V)
+    need = gpu.workspace_bytes(gpu.DTYPE_BF16, N, V, V)
+    plain = (256 << 10) + N * (2 * ((V + 63) & ~63) * 8 + 6 * 16 * 256 * 4 + 16 * 64 + 2 * 40 * 8)
+    assert plain < need
+    for nbytes in (need, plain):
+        ws = gpu.Workspace((nbytes + 255) & ~255)
+        check(gpu, oracle, x, u, 0.8, 0.95, workspace=ws, want_probs=False)
+        check(gpu, oracle, x, u, 0.8, 0.95, workspace=ws)
+        ws.free()
+    check(gpu, oracle, x, u, 0.8, 0.95, noalloc=True, want_probs=False)
+    u = u[:, :9000]
+    check(gpu, oracle, x, u, 0.8, 0.95, noalloc=True, want_probs=False)
+    check(gpu, oracle, x, u, 0.8, 0.95, workspace=(None, 0), want_probs=False)
