@@ -183,21 +183,21 @@ size_t routed_workspace_bytes(const d3s::SampleArgs &a, d3s::Dtype dt) {
   return 0;
 }
 
-/* the workspace with which rows go to the selecting kernels (k up to 4096),
- * or the sorting kernels gather only the keys they need (after the counters'
- * block); 0 when neither takes the call.  It is not required: without it the
- * streaming kernel takes the rows, or the sorting kernels all their keys (the
- * same bits).  one_row: enough for the rows one after the other. */
+/* the workspace with which rows go to the selecting kernels (k up to 4096) or
+ * the wide nucleus kernels (larger k, ids only), or the sorting kernels gather
+ * only the keys they need (after the counters' block); 0 when none takes the
+ * call.  It is not required: without it the streaming kernel takes the rows, or
+ * the sorting kernels all their keys (the same bits).  one_row: enough for the
+ * rows one after the other. */
 size_t optional_workspace_bytes(const d3s::SampleArgs &a, d3s::Dtype dt, bool one_row) {
   const size_t off = d3s::split_counter_bytes();
-  if (a.k > d3s::generic_max_k()) {
-    if ((a.flags & D3S_FLAG_GENERIC) == 0u && a.vocab <= d3s::topp_max_vocab()) return 0;
-    return one_row ? 0 : off + d3s::bigk_workspace_bytes(a, dt, BIGK_WS_CAP);
-  }
-  if ((a.flags & D3S_FLAG_GENERIC) != 0u || !a.opgraph || a.vocab <= d3s::topp_max_vocab()) return 0;
+  const bool generic = (a.flags & D3S_FLAG_GENERIC) != 0u, sorts = a.k > d3s::generic_max_k();
+  if (!a.opgraph || a.vocab <= d3s::topp_max_vocab() || (generic && !sorts)) return 0;
   if (d3s::split_segments(a, dt) > 0 || (a.k <= 64 && a.vocab <= d3s::wide_max_vocab(dt))) return 0;
   if (d3s::sel_takes(a)) return off + d3s::sel_workspace_bytes(a, dt, one_row);
-  return off + d3s::bigk_workspace_bytes(a, dt, one_row ? 1 : BIGK_WS_CAP);
+  const size_t sort = sorts && one_row ? 0 : d3s::bigk_workspace_bytes(a, dt, one_row ? 1 : BIGK_WS_CAP);
+  const size_t nucleus = !generic && d3s::nucleus_takes(a) ? d3s::nucleus_workspace_bytes(a, dt, one_row) : 0;
+  return off + (nucleus > sort ? nucleus : sort);
 }
 
 /* Where a call's workspace comes from: the block the library keeps for the
@@ -251,10 +251,13 @@ int sample_routed(const d3s::SampleArgs &a, d3s::Dtype dt, hipStream_t s, Ws w) 
       w.ptr = d3s::stream_workspace_optional(s, want);
       w.bytes = w.ptr ? want : 0;
     }
-    if (a.k <= d3s::generic_max_k() && w.ptr && w.bytes > off &&
-        (d3s::launch_select(a, dt, (char *)w.ptr + off, w.bytes - off, s) ||
-         (a.k > 64 && d3s::launch_bigk(a, dt, (char *)w.ptr + off, w.bytes - off, s))))
-      return launched();
+    if (w.ptr && w.bytes > off) {
+      void *p = (char *)w.ptr + off;
+      const size_t bytes = w.bytes - off;
+      if (d3s::launch_select(a, dt, p, bytes, s) || (!generic && d3s::launch_nucleus(a, dt, p, bytes, s)) ||
+          (a.k <= d3s::generic_max_k() && a.k > 64 && d3s::launch_bigk(a, dt, p, bytes, s)))
+        return launched();
+    }
   }
   if (a.k > d3s::generic_max_k()) { /* the sorting kernels, their keys after the counters' block */
     if (!w.ptr && w.lazy) {

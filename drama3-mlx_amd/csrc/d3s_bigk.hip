@@ -56,19 +56,6 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-/* the wave's lanes whose d has the same low `bits` bits as this lane's
- * (among the lanes in `live`), by one ballot per bit */
-template <int BITS>
-__device__ __forceinline__ uint64_t wave_peers(uint32_t d, uint64_t live) {
-  uint64_t peers = live;
-#pragma unroll
-  for (int b = 0; b < BITS; b++) {
-    const uint64_t bb = __ballot((d >> b) & 1u);
-    peers &= ((d >> b) & 1u) ? bb : ~bb;
-  }
-  return peers;
-}
-
 /* block sum of per-thread fixed-point values, exact modulo 2^64 (the
  * oracle's integer sums); opens with a barrier (the scratch may still be
  * being read) */

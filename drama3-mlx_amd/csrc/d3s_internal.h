@@ -162,6 +162,11 @@ size_t topp_workspace_bytes(const SampleArgs &a);
 bool launch_select(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hipStream_t s);
 bool sel_takes(const SampleArgs &a);
 size_t sel_workspace_bytes(const SampleArgs &a, Dtype dt, bool one_row);
+/* Launch the wide nucleus kernels (ids only, op graph's order, k > 4096, rows
+ * longer than the nucleus kernel takes): no sort.  Workspace as launch_select's. */
+bool launch_nucleus(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hipStream_t s);
+bool nucleus_takes(const SampleArgs &a);
+size_t nucleus_workspace_bytes(const SampleArgs &a, Dtype dt, bool one_row);
 /* Launch the streaming generic kernel (any V, k <= generic_max_k()). */
 bool launch_generic(const SampleArgs &a, Dtype dt, hipStream_t s);
 int generic_max_k();

@@ -88,6 +88,19 @@ __device__ __forceinline__ uint32_t bk_digit(uint64_t key, int pass) {
   return (uint32_t)((~key) >> (32 + 8 * pass)) & 0xffu;
 }
 
+/* the wave's lanes whose d has the same low `bits` bits as this lane's
+ * (among the lanes in `live`), by one ballot per bit */
+template <int BITS>
+__device__ __forceinline__ uint64_t wave_peers(uint32_t d, uint64_t live) {
+  uint64_t peers = live;
+#pragma unroll
+  for (int b = 0; b < BITS; b++) {
+    const uint64_t bb = __ballot((d >> b) & 1u);
+    peers &= ((d >> b) & 1u) ? bb : ~bb;
+  }
+  return peers;
+}
+
 /* sum over the wave of per-lane 64-bit values, exact modulo 2^64 (three
  * 24-bit parts, each summed in 32 bits): a thread's partial sum over a long
  * segment of terms near 2^40 can pass the shared wave sum's 2^45 */
@@ -241,6 +254,17 @@ __device__ __forceinline__ bool sel_t_easy(float T) {
 
 /* the bucket of z = x - m <= 0 (-inf: the last) */
 __device__ __forceinline__ int sel_bucket(float z) { return (int)fminf(z * -SEL_SCALE, (float)(SEL_NB - 1)); }
+
+/* a bound every logit of the buckets up to b reaches: (b + 1) / SEL_SCALE below
+ * m, with room for the roundings of x, of x - m and of this bound */
+__device__ __forceinline__ float sel_logit_bound(float M, float T, int b) {
+  const float ninf = -__builtin_inff();
+  if (b >= SEL_NB - 1 || !(T < __builtin_inff())) return ninf;
+  const float xc = M - ((float)(b + 1) * (1.0f / SEL_SCALE)) * 1.0001f;
+  float Lc = (xc - (fabsf(M) + fabsf(xc) + 1.0f) * 0x1p-20f) * T;
+  Lc = Lc - fabsf(Lc) * 0x1p-20f;
+  return Lc >= -0x1.fffffep127f ? Lc : ninf;
+}
 
 }  // namespace
 

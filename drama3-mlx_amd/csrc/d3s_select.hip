@@ -136,11 +136,11 @@ __global__ __launch_bounds__(SEL_T) void k_sel_hist(SampleArgs a, SelLayout L) {
   __syncthreads();
   const uint4 c = ((const uint4 *)cnt)[tid];
   ((uint4 *)(L.cnt + at * SEL_NB))[tid] = c;
-  uint32_t g = c.x + c.y + c.z + c.w;
+  uint32_t g = c.x + c.y + c.z + c.w; /* (the group's count; the wide nucleus path takes none) */
   g += dpp_u<0xb1, 0xf>(0u, g);   /* quad_perm [1,0,3,2] */
   g += dpp_u<0x4e, 0xf>(0u, g);   /* quad_perm [2,3,0,1] */
   g += dpp_u<0x141, 0xf>(0u, g);  /* row_half_mirror: the other four of the eight */
-  if (tid % (SEL_G / PER) == 0) L.group[at * SEL_NG + tid / (SEL_G / PER)] = g;
+  if (!SUMS && tid % (SEL_G / PER) == 0) L.group[at * SEL_NG + tid / (SEL_G / PER)] = g;
   if (tid == 0) {
 #pragma unroll
     for (int w = 1; w < SEL_NW; w++) acc += sum[w];
@@ -216,17 +216,9 @@ __global__ __launch_bounds__(SEL_T) void k_sel_gather(SampleArgs a, SelLayout L,
   __syncthreads();
   const uint32_t fin = before + wave_scan_add_u32(lane < SEL_G ? fine[lane] : 0u);
   const int tb = tg * SEL_G + (int)__builtin_ctzll(__ballot(fin >= k) | (1ull << (SEL_G - 1)));
-  /* every logit of the buckets up to tb reaches Lc: (tb + 1) / SEL_SCALE below
-   * m, with room for the roundings of x, of x - m and of this bound (a few
-   * elements below them may as well: the set holds every element above any of
-   * its own, which is all that the ranking asks) */
-  float Lc = -__builtin_inff();
-  if (tb < SEL_NB - 1 && T < __builtin_inff()) {
-    const float xc = M - ((float)(tb + 1) * (1.0f / SEL_SCALE)) * 1.0001f;
-    Lc = (xc - (fabsf(M) + fabsf(xc) + 1.0f) * 0x1p-20f) * T;
-    Lc = Lc - fabsf(Lc) * 0x1p-20f;
-    if (!(Lc >= -0x1.fffffep127f)) Lc = -__builtin_inff();
-  }
+  /* (a few elements below bucket tb may reach Lc as well: the set holds every
+   * element above any of its own, which is all that the ranking asks) */
+  const float Lc = sel_logit_bound(M, T, tb);
   auto pick = [&](const auto &v, uint32_t ok) -> uint32_t {
     uint32_t m = 0u;
 #pragma unroll

@@ -1,5 +1,6 @@
 """The selecting kernels (64 < k <= 4096 on rows longer than 8192, and small k
-on rows wider than the segmented kernel's) against the oracle, bit for bit:
+on rows wider than the segmented kernel's) and the wide nucleus kernels (k >
+4096, ids only) against the oracle, bit for bit:
 row lengths at segment and chunk edges, row starts off 16 bytes, k at its
 limits, ties across the k-th place, rows the kernels leave to the generic
 procedure, and every workspace mode."""
@@ -154,7 +155,7 @@ def test_captured_and_replayed(gpu, oracle, own_workspace):
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("sigma", [0.1, 1.0, 3.0, 8.0])
 def test_ids_only_large_k_gathers_the_kept_ranks(gpu, oracle, dtype, sigma):
-    """k > 4096, ids only (the sorting kernels take the ranks top-p can keep):
+    """k > 4096, ids only (the wide nucleus kernels):
     every top_p from 0 to beyond 1, temperatures, banned indices, strides"""
     rng = np.random.default_rng([int(sigma * 10), dtype == "f32"])
     V = 24007
@@ -202,8 +203,8 @@ def test_ids_only_large_k_special_rows(gpu, oracle):
 
 
 def test_sorting_workspace_modes_agree(gpu, oracle):
-    """the query's workspace, one that holds only the plain sort's keys (what
-    the call requires), and the allocation-free entry point"""
+    """the query's workspace, one that holds only the sort's keys (what the call
+    requires), and the allocation-free entry point"""
     rng = np.random.default_rng(14)
     N, V = 3, 40009
     x, u = rows(rng, N, V, "bf16"), oracle.uniform(9, 1, N, V)
