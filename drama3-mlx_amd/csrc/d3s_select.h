@@ -150,33 +150,34 @@ __device__ __forceinline__ SelRun sel_run(const SampleArgs &a, const SelLayout &
   return r;
 }
 
-/* SEL_U 16-byte loads a lane from chunk `base` of the run on (zeros past it) */
-__device__ __forceinline__ void sel_load(const SelRun &r, int base, uint4 (&q)[SEL_U]) {
+/* U 16-byte loads a lane from chunk `base` of the run on (zeros past it) */
+template <int U>
+__device__ __forceinline__ void sel_load(const SelRun &r, int base, uint4 (&q)[U]) {
 #pragma unroll
-  for (int u = 0; u < SEL_U; u++) {
+  for (int u = 0; u < U; u++) {
     const int c = base + u * WAVE + lane_id();
     q[u] = c < r.c1 ? r.src[c] : make_uint4(0u, 0u, 0u, 0u);
   }
 }
 
 /* fn(v, p0, ok) for every chunk of the run, `first` the loads of its first
- * SEL_U rows of chunks (issued by the caller ahead of whatever it waits for):
+ * U rows of chunks (issued by the caller ahead of whatever it waits for):
  * v the EPC logits (-inf outside the row and at the banned index), p0 the
  * first one's position, ok the bits of those within the run and the row.
  * Every lane calls fn. */
-template <bool BF16, class Fn>
-__device__ __forceinline__ void sel_chunks(const SelRun &r, int V, int banned, const uint4 (&first)[SEL_U], Fn &&fn) {
+template <bool BF16, int U, class Fn>
+__device__ __forceinline__ void sel_chunks(const SelRun &r, int V, int banned, const uint4 (&first)[U], Fn &&fn) {
   constexpr int EPC = BF16 ? 8 : 4;
   const int lane = lane_id();
-  uint4 q[SEL_U], next[SEL_U];
+  uint4 q[U], next[U];
 #pragma unroll
-  for (int u = 0; u < SEL_U; u++) q[u] = first[u];
+  for (int u = 0; u < U; u++) q[u] = first[u];
   /* one copy of fn's code: the launch's instruction fetch costs more than the
    * register moves of a rolled loop */
 #pragma unroll 1
-  for (int base = r.c0; base < r.c1; base += SEL_U * WAVE) {
-    sel_load(r, base + SEL_U * WAVE, next);
-    const int end = min(r.c1, base + SEL_U * WAVE);
+  for (int base = r.c0; base < r.c1; base += U * WAVE) {
+    sel_load(r, base + U * WAVE, next);
+    const int end = min(r.c1, base + U * WAVE);
 #pragma unroll 1
     for (int cw = base; cw < end; cw += WAVE) { /* cw uniform: the 64 chunks' first */
       const int p0 = (cw + lane) * EPC - r.off, f0 = cw * EPC - r.off;
@@ -197,10 +198,10 @@ __device__ __forceinline__ void sel_chunks(const SelRun &r, int V, int banned, c
       }
       fn(v, p0, ok);
 #pragma unroll
-      for (int u = 0; u + 1 < SEL_U; u++) q[u] = q[u + 1];
+      for (int u = 0; u + 1 < U; u++) q[u] = q[u + 1];
     }
 #pragma unroll
-    for (int u = 0; u < SEL_U; u++) q[u] = next[u];
+    for (int u = 0; u < U; u++) q[u] = next[u];
   }
 }
 
