@@ -473,7 +473,8 @@ int ras_call(const void *logits, int dtype, int64_t n_rows, int64_t vocab, int64
   int32_t *ri = retry_out ? retry_out : (int32_t *)((char *)p + idx_off);
   r.first.ids = fi;
   r.retry.ids = ri;
-  const Ws w = fixed_ws(p, need, mode == WsMode::Caller ? D3S_ERR_WORKSPACE : D3S_ERR_NOMEM);
+  /* (the draws' part alone: what lies past it is the retry's indices) */
+  const Ws w = fixed_ws(p, retry_out ? need : idx_off, mode == WsMode::Caller ? D3S_ERR_WORKSPACE : D3S_ERR_NOMEM);
   int rc = sample_routed(r.first, dt, s, w);
   if (rc == D3S_OK) rc = sample_routed(r.retry, dt, s, w);
   if (rc != D3S_OK) return rc;
@@ -587,8 +588,9 @@ int linear_sample_call(const uint16_t *x, const uint16_t *w, int64_t n_rows, int
   d3s::launch_linear(la, s);
   const int rc = launched();
   if (rc != D3S_OK) return rc;
+  /* (the sample's part alone: what lies past it is the logits) */
   return sample_routed(a, d3s::DT_BF16, s,
-                       fixed_ws(p, need, mode == WsMode::Caller ? D3S_ERR_WORKSPACE : D3S_ERR_NOMEM));
+                       fixed_ws(p, y ? need : y_off, mode == WsMode::Caller ? D3S_ERR_WORKSPACE : D3S_ERR_NOMEM));
 }
 
 }  // namespace

@@ -220,3 +220,21 @@ def test_sorting_workspace_modes_agree(gpu, oracle):
     u = u[:, :9000]
     check(gpu, oracle, x, u, 0.8, 0.95, noalloc=True, want_probs=False)
     check(gpu, oracle, x, u, 0.8, 0.95, workspace=(None, 0), want_probs=False)
+
+
+@pytest.mark.parametrize("k", [100, 6000, 20001])
+def test_head_with_its_logits_in_the_workspace(gpu, k):
+    """the heads' logits lie in the workspace behind the sample's part when the
+    caller keeps none: the routes that use a workspace when they have one must
+    not take that part for theirs"""
+    rng = np.random.default_rng(k)
+    N, K, V = 8, 128, 20001
+    x = W.f32_to_bf16_bits(rng.standard_normal((N, K)).astype(np.float32))
+    w = W.f32_to_bf16_bits((rng.standard_normal((V, K)) * 0.2).astype(np.float32))
+    u = rng.random((N, k)).astype(np.float32)
+    for want_probs in (True, False):
+        kept = gpu.linear_sample_bf16(x, w, u, 1.0, 0.9, want_probs=want_probs)
+        got = gpu.linear_sample_bf16(x, w, u, 1.0, 0.9, want_probs=want_probs, keep_logits=False)
+        assert kept["rc"] == 0 and got["rc"] == 0
+        for name in ("ids", "cand", "probs") if want_probs else ("ids",):
+            assert np.array_equal(kept[name], got[name]), name
