@@ -83,21 +83,22 @@ void *stream_workspace(hipStream_t s, size_t bytes) {
   return p;
 }
 
-/* stream_workspace for a route that another kernel can take without one: no
- * allocation while the stream is being captured, nothing that another
+/* stream_workspace for a route that another kernel can take without one: none
+ * while the stream is being captured (a graph may be replayed beside other
+ * calls on the stream, or outlive the block), and no allocation that another
  * stream's capture forbids (the block is cleared by a kernel on `s`) */
 void *stream_workspace_optional(hipStream_t s, size_t bytes) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-  std::lock_guard<std::mutex> lock(g_ws_mutex);
-  const Key key{dev, (uintptr_t)s};
-  Block &b = g_ws[key];
-  if (b.bytes >= bytes) return b.ptr;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();
     return nullptr;
   }
+  std::lock_guard<std::mutex> lock(g_ws_mutex);
+  const Key key{dev, (uintptr_t)s};
+  Block &b = g_ws[key];
+  if (b.bytes >= bytes) return b.ptr;
   const size_t want = (bytes + (1u << 20) - 1) & ~(size_t)((1u << 20) - 1); /* whole MiB */
   void *p = nullptr;
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;

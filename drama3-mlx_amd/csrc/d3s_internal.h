@@ -100,8 +100,7 @@ void launch_ras_select(const RasArgs &r, const int32_t *first, const int32_t *re
  * outgrows is kept (a call on another thread may still be enqueueing on it)
  * until release_stream_workspace.  Null when the allocation fails. */
 void *stream_workspace(hipStream_t s, size_t bytes);
-/* The same for a route that can do without: null while `s` is being captured
- * (unless the block it has is large enough). */
+/* The same for a route that can do without: null while `s` is being captured. */
 void *stream_workspace_optional(hipStream_t s, size_t bytes);
 /* Waits for the stream, then frees its block and the blocks it outgrew. */
 int release_stream_workspace(hipStream_t s);

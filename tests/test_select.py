@@ -113,11 +113,13 @@ def test_workspace_modes_agree(gpu, oracle):
     check(gpu, oracle, x, u, 0.8, 0.95, flags=gpu.FLAG_GENERIC)
 
 
-@pytest.mark.parametrize("own_workspace", [True, False])
+@pytest.mark.parametrize("own_workspace", [True, False, None])
 def test_captured_and_replayed(gpu, oracle, own_workspace):
     """d3s_sample_ws (the selecting kernels) and d3s_sample on a stream that has
     no block yet (nothing is allocated under capture: the streaming kernel),
-    captured and replayed with new inputs between the replays"""
+    captured and replayed with new inputs between the replays; None: a stream
+    whose block is large enough, released before the replays (a graph does not
+    hold it)"""
     import ctypes
     import hiprt
     H = hiprt.hip()
@@ -125,6 +127,10 @@ def test_captured_and_replayed(gpu, oracle, own_workspace):
     bx, bu, bids = hiprt.DeviceBuffer(4 * N * V), hiprt.DeviceBuffer(4 * N * k), hiprt.DeviceBuffer(4 * N)
     s = hiprt.Stream()
     ws = gpu.Workspace(gpu.workspace_bytes(gpu.DTYPE_F32, N, V, k)) if own_workspace else None
+    if own_workspace is None:
+        bx.upload(rows(np.random.default_rng(9), N, V, "f32"))
+        bu.upload(oracle.uniform(1, 9, N, k))
+        assert gpu.sample_raw(bx.ptr, gpu.DTYPE_F32, N, V, V, bu.ptr, k, 0.8, 0.9, None, bids.ptr, stream=s.ptr) == 0
     hiprt.synchronize()
     graph, exe = ctypes.c_void_p(), ctypes.c_void_p()
     hiprt.check(H.hipStreamBeginCapture(s.ptr, 0), "begin capture")
@@ -133,6 +139,9 @@ def test_captured_and_replayed(gpu, oracle, own_workspace):
     hiprt.check(H.hipStreamEndCapture(s.ptr, ctypes.byref(graph)), "end capture")
     assert rc == 0
     assert set(hiprt.graph_node_types(graph)) == {"kernel"}
+    if own_workspace is None:  # the streaming kernel alone
+        assert len(hiprt.graph_node_types(graph)) == 1
+        assert gpu.lib().d3s_stream_workspace_release(s.ptr) == 0
     hiprt.check(H.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0), "instantiate")
     try:
         for rep in range(4):
