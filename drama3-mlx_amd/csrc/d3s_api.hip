@@ -356,8 +356,10 @@ int sample_call(const void *logits, int dtype, int64_t n_rows, int64_t vocab, in
   if (mode == WsMode::Caller) {
     const int rc = check_caller_ws(ws, ws_bytes, need);
     if (rc != D3S_OK) return rc;
-    /* (a workspace the route does not require is used where it can be) */
-    const bool use = need > 0 || (ws && (uintptr_t)ws % 256u == 0u && optional_workspace_bytes(a, dt, true) > 0);
+    /* (a workspace the route does not require is used where it can be, and
+     * where the size query tells of it: k > 64) */
+    const bool use = need > 0 || (k > 64 && ws && (uintptr_t)ws % 256u == 0u &&
+                                  optional_workspace_bytes(a, dt, true) > 0);
     return sample_routed(a, dt, s, fixed_ws(use ? ws : nullptr, (size_t)ws_bytes, D3S_ERR_WORKSPACE));
   }
   void *p = nullptr;

@@ -117,9 +117,10 @@ int d3s_sample(const void *logits, int dtype, int64_t n_rows, int64_t vocab, int
  * the call's route keeps no state in device memory), or a negative status for
  * arguments d3s_sample rejects.  The need depends on dtype, n_rows, vocab, k
  * and flags (and on D3_NO_FUSED_SAMPLER only through the route, not the size).
- * For 64 < k <= 4096 on rows longer than 8192 it is the size with which the
+ * For 64 < k <= 16384 on rows longer than 8192 it is the size with which the
  * rows are spread over the chip; a smaller workspace, or none, is accepted
- * there and gives the same results more slowly.
+ * there and gives the same results more slowly (for larger k: one that holds
+ * a row's sort keys).
  * Replaces the one-time set-up of sample_kernel_call (src/sampling.c:142-157). */
 int64_t d3s_sample_workspace_bytes(int dtype, int64_t n_rows, int64_t vocab, int k, unsigned flags);
 

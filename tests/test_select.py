@@ -247,3 +247,19 @@ def test_head_with_its_logits_in_the_workspace(gpu, k):
         assert kept["rc"] == 0 and got["rc"] == 0
         for name in ("ids", "cand", "probs") if want_probs else ("ids",):
             assert np.array_equal(kept[name], got[name]), name
+
+
+def test_small_k_leaves_the_workspace(gpu, oracle):
+    """k up to 64: the size query says 0, and a workspace given all the same is
+    not written"""
+    import hiprt
+    N, V, k = 2, 700001, 20
+    x, u = rows(np.random.default_rng(15), N, V, "f32"), oracle.uniform(5, 1, N, k)
+    assert gpu.workspace_bytes(gpu.DTYPE_F32, N, V, k) == 0
+    fill = np.full(16 << 18, 0x5a5a5a5a, np.uint32)
+    ws, bx, bu, bids = hiprt.to_device(fill), hiprt.to_device(x), hiprt.to_device(u), hiprt.DeviceBuffer(4 * N)
+    assert gpu.sample_raw(bx.ptr, gpu.DTYPE_F32, N, V, V, bu.ptr, k, 0.8, 0.9, None, bids.ptr,
+                          workspace=(ws.ptr, fill.nbytes)) == 0
+    hiprt.synchronize()
+    assert np.array_equal(bids.download((N,), np.int32), oracle.sample(x, u, 0.8, 0.9)["ids"])
+    assert np.array_equal(ws.download(fill.shape, np.uint32), fill)
