@@ -434,7 +434,7 @@ def other_configs(reps):
             f"({100 * gbs / HBM_PEAK_GBS:.1f} % of HBM peak)")
         del lg, u
     # C4's rows with top-k disabled (k = V, the op graph's full argsort,
-    # src/sampling.c:33-35): the sorting kernel
+    # src/sampling.c:33-35), ids only: the wide nucleus kernels
     w = W.make("C4", seed=5, uniforms=False)
     x = w["logits"]
     N, Vc = x.shape
