@@ -10,10 +10,11 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <atomic>
 #include <map>
 #include <memory>
 #include <mutex>
-#include <utility>
+#include <tuple>
 #include <vector>
 
 #include "../../include/d3s_sampler.h"
@@ -34,7 +35,17 @@ struct Block {
   void *ptr = nullptr;
   size_t bytes = 0;
 };
-using Key = std::pair<int, uintptr_t>; /* (device, stream) */
+using Key = std::tuple<int, uintptr_t, uint64_t>; /* (device, stream, thread of a per-thread stream) */
+/* hipStreamPerThread is one handle for every thread's own stream: its calls
+ * run beside each other, so each thread has a block and a lock of its own
+ * (numbers are never used twice: a later thread cannot take the block of one
+ * whose work may still run) */
+Key stream_key(int dev, hipStream_t s) {
+  static std::atomic<uint64_t> threads{0};
+  thread_local uint64_t mine = 0;
+  if (s == hipStreamPerThread && mine == 0) mine = ++threads;
+  return Key{dev, (uintptr_t)s, s == hipStreamPerThread ? mine : 0};
+}
 std::mutex g_ws_mutex;
 std::map<Key, Block> g_ws;
 /* blocks a stream has outgrown: a call on another thread may have taken one
@@ -56,7 +67,7 @@ std::unique_lock<std::recursive_mutex> stream_call_lock(hipStream_t s) {
   std::recursive_mutex *m = nullptr;
   {
     std::lock_guard<std::mutex> lock(g_ws_mutex);
-    std::unique_ptr<std::recursive_mutex> &p = g_call_locks[Key{dev, (uintptr_t)s}];
+    std::unique_ptr<std::recursive_mutex> &p = g_call_locks[stream_key(dev, s)];
     if (!p) p = std::make_unique<std::recursive_mutex>();
     m = p.get();
   }
@@ -67,7 +78,7 @@ void *stream_workspace(hipStream_t s, size_t bytes) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return nullptr;
   std::lock_guard<std::mutex> lock(g_ws_mutex);
-  const Key key{dev, (uintptr_t)s};
+  const Key key = stream_key(dev, s);
   Block &b = g_ws[key];
   if (b.bytes >= bytes) return b.ptr;
   const size_t want = (bytes + (1u << 20) - 1) & ~(size_t)((1u << 20) - 1); /* whole MiB */
@@ -96,7 +107,7 @@ void *stream_workspace_optional(hipStream_t s, size_t bytes) {
     return nullptr;
   }
   std::lock_guard<std::mutex> lock(g_ws_mutex);
-  const Key key{dev, (uintptr_t)s};
+  const Key key = stream_key(dev, s);
   Block &b = g_ws[key];
   if (b.bytes >= bytes) return b.ptr;
   const size_t want = (bytes + (1u << 20) - 1) & ~(size_t)((1u << 20) - 1); /* whole MiB */
@@ -121,7 +132,7 @@ int release_stream_workspace(hipStream_t s) {
   if (hipGetDevice(&dev) != hipSuccess) return D3S_ERR_LAUNCH;
   if (hipStreamSynchronize(s) != hipSuccess) return D3S_ERR_LAUNCH;
   std::lock_guard<std::mutex> lock(g_ws_mutex);
-  const Key key{dev, (uintptr_t)s};
+  const Key key = stream_key(dev, s);
   auto it = g_ws.find(key);
   if (it != g_ws.end()) {
     if (it->second.ptr) (void)hipFree(it->second.ptr);

@@ -20,6 +20,7 @@ def hip():
         H.hipMemcpy.argtypes = [vp, vp, sz, i32]
         H.hipMemcpyAsync.argtypes = [vp, vp, sz, i32, vp]
         H.hipMemset.argtypes = [vp, i32, sz]
+        H.hipMemGetInfo.argtypes = [ctypes.POINTER(sz), ctypes.POINTER(sz)]
         H.hipDeviceSynchronize.argtypes = []
         H.hipGetDeviceCount.argtypes = [ctypes.POINTER(i32)]
         H.hipStreamCreate.argtypes = [ctypes.POINTER(vp)]
@@ -41,7 +42,7 @@ def hip():
         H.hipGraphDestroy.argtypes = [vp]
         H.hipGraphGetNodes.argtypes = [vp, ctypes.POINTER(vp), ctypes.POINTER(sz)]
         H.hipGraphNodeGetType.argtypes = [vp, ctypes.POINTER(i32)]
-        for f in ("hipMalloc", "hipFree", "hipMemcpy", "hipMemcpyAsync", "hipMemset",
+        for f in ("hipMalloc", "hipFree", "hipMemcpy", "hipMemcpyAsync", "hipMemset", "hipMemGetInfo",
                   "hipDeviceSynchronize", "hipGetDeviceCount", "hipStreamCreate",
                   "hipStreamDestroy", "hipStreamSynchronize", "hipStreamWaitEvent", "hipEventCreate", "hipEventDestroy",
                   "hipEventRecord", "hipEventSynchronize", "hipEventElapsedTime",
@@ -68,6 +69,13 @@ def device_count():
     n = ctypes.c_int(0)
     rc = hip().hipGetDeviceCount(ctypes.byref(n))
     return n.value if rc == 0 else 0
+
+
+def free_memory():
+    """free bytes of the current device's memory"""
+    free, total = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    check(hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)), "hipMemGetInfo")
+    return free.value
 
 
 class DeviceBuffer:

@@ -23,7 +23,8 @@
  * d3s_linear_sample_bf16) are a convenience that takes the workspace from a
  * block the library keeps per (device, stream), allocated on the stream's
  * first call that needs one (the NULL stream is one such stream for every
- * thread); d3s_stream_workspace_release frees a stream's block.  Such calls
+ * thread; hipStreamPerThread is a stream, and a block, of each thread's own);
+ * d3s_stream_workspace_release frees a stream's block.  Such calls
  * on one stream from several host threads each enqueue all their launches
  * before the next one starts (a lock per (device, stream)): their launches
  * never interleave on the block.
@@ -146,8 +147,9 @@ int d3s_workspace_init(void *workspace, int64_t bytes, void *stream);
 /* Frees the block the library keeps for `stream` on the current device
  * (d3s_sample, d3s_sample_ras and d3s_linear_sample_bf16 without _ws), after
  * waiting for the stream.  For a stream about to be destroyed, or to give the
- * memory back; the next call on the stream that needs a block allocates a new
- * one.  No call may use the stream meanwhile. */
+ * memory back (hipStreamPerThread: by the thread itself, before it ends); the
+ * next call on the stream that needs a block allocates a new one.  No call may
+ * use the stream meanwhile. */
 int d3s_stream_workspace_release(void *stream);
 
 /* d3s_sample without any allocation, for callers that cannot allocate device
