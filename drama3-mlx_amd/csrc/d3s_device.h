@@ -81,6 +81,26 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
   return ((uint64_t)hi << 24) + lo;
 }
 
+/* sum over the wave of per-lane 64-bit values, exact modulo 2^64 (three
+ * 24-bit parts, each summed in 32 bits): for a thread's share of a long row,
+ * whose terms near 2^40 can pass 2^45 (wave_sum_u64 wraps from 2^50 on: 1024
+ * such terms a lane) */
+__device__ __forceinline__ uint64_t wave_sum_mod64(uint64_t v) {
+  const uint32_t p0 = wave_sum_u32((uint32_t)(v & 0xffffffu));
+  const uint32_t p1 = wave_sum_u32((uint32_t)((v >> 24) & 0xffffffu));
+  const uint32_t p2 = wave_sum_u32((uint32_t)(v >> 48));
+  return (uint64_t)p0 + ((uint64_t)p1 << 24) + ((uint64_t)p2 << 48);
+}
+
+/* inclusive prefix sum over the wave of per-lane 64-bit values, exact
+ * modulo 2^64 */
+__device__ __forceinline__ uint64_t wave_scan_mod64(uint64_t v) {
+  const uint32_t p0 = wave_scan_add_u32((uint32_t)(v & 0xffffffu));
+  const uint32_t p1 = wave_scan_add_u32((uint32_t)((v >> 24) & 0xffffffu));
+  const uint32_t p2 = wave_scan_add_u32((uint32_t)(v >> 48));
+  return (uint64_t)p0 + ((uint64_t)p1 << 24) + ((uint64_t)p2 << 48);
+}
+
 /* inclusive prefix sum over the wave of per-lane values below 2^40 (lane i
  * gets lanes 0..i), exact: the low 24 bits and the rest scanned apart */
 __device__ __forceinline__ uint64_t wave_scan_u64(uint64_t v) {

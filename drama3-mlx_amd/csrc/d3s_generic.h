@@ -118,7 +118,7 @@ __device__ __forceinline__ void generic_tail_opgraph(const SampleArgs &a, const 
     if (r < k && r < cut) ks += d3s_fix40(d3s_expf(key_x(glist[r]) - v0));
   }
   {
-    const uint64_t w = wave_sum_u64(ks);
+    const uint64_t w = wave_sum_mod64(ks);
     __syncthreads();
     if (lane == 0) {
       sh_lo[wid] = (uint32_t)w;
@@ -223,7 +223,7 @@ __device__ __forceinline__ void generic_row_src(const SampleArgs &a, const int r
   uint64_t acc = 0;
   for (int i = tid; i < V; i += GBLOCK) acc += d3s_fix40(d3s_expf(xat(i) - M));
   {
-    const uint64_t w = wave_sum_u64(acc);
+    const uint64_t w = wave_sum_mod64(acc);
     if (lane == 0) {
       sh_lo[wid] = (uint32_t)w;
       sh_hi[wid] = (uint32_t)(w >> 32);

@@ -101,25 +101,6 @@ __device__ __forceinline__ uint64_t wave_peers(uint32_t d, uint64_t live) {
   return peers;
 }
 
-/* sum over the wave of per-lane 64-bit values, exact modulo 2^64 (three
- * 24-bit parts, each summed in 32 bits): a thread's partial sum over a long
- * segment of terms near 2^40 can pass the shared wave sum's 2^45 */
-__device__ __forceinline__ uint64_t wave_sum_mod64(uint64_t v) {
-  const uint32_t p0 = wave_sum_u32((uint32_t)(v & 0xffffffu));
-  const uint32_t p1 = wave_sum_u32((uint32_t)((v >> 24) & 0xffffffu));
-  const uint32_t p2 = wave_sum_u32((uint32_t)(v >> 48));
-  return (uint64_t)p0 + ((uint64_t)p1 << 24) + ((uint64_t)p2 << 48);
-}
-
-/* inclusive prefix sum over the wave of per-lane 64-bit values, exact
- * modulo 2^64 */
-__device__ __forceinline__ uint64_t wave_scan_mod64(uint64_t v) {
-  const uint32_t p0 = wave_scan_add_u32((uint32_t)(v & 0xffffffu));
-  const uint32_t p1 = wave_scan_add_u32((uint32_t)((v >> 24) & 0xffffffu));
-  const uint32_t p2 = wave_scan_add_u32((uint32_t)(v >> 48));
-  return (uint64_t)p0 + ((uint64_t)p1 << 24) + ((uint64_t)p2 << 48);
-}
-
 __device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int l) {
   return ((uint64_t)readlane_u((uint32_t)(v >> 32), l) << 32) | readlane_u((uint32_t)v, l);
 }

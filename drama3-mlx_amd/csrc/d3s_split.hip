@@ -94,7 +94,7 @@ __device__ __forceinline__ float split_exact_lse(const SampleArgs &a, int row, f
 #pragma unroll
     for (int e = 0; e < EPC; e++) acc += d3s_fix40_exp(x[e] - M); /* (0 for -inf, outside the row as well) */
   });
-  const uint64_t w = wave_sum_u64(acc);
+  const uint64_t w = wave_sum_mod64(acc);
   if (lane_id() == 0) {
     S.slo[wid] = (uint32_t)w;
     S.shi[wid] = (uint32_t)(w >> 32);
