@@ -34,7 +34,12 @@ namespace {
 struct Block {
   void *ptr = nullptr;
   size_t bytes = 0;
+  int denied = 0; /* requests left that do not ask for more memory */
 };
+constexpr int DENIED_CALLS = 255;
+/* a block grows by doubling up to what the kernels that share out rows take
+ * for a launch (then launches of fewer rows); a call that needs more gets it */
+constexpr size_t WS_CAP = (size_t)257 << 20;
 using Key = std::tuple<int, uintptr_t, uint64_t>; /* (device, stream, thread of a per-thread stream) */
 /* hipStreamPerThread is one handle for every thread's own stream: its calls
  * run beside each other, so each thread has a block and a lock of its own
@@ -74,6 +79,44 @@ std::unique_lock<std::recursive_mutex> stream_call_lock(hipStream_t s) {
   return std::unique_lock<std::recursive_mutex>(*m);
 }
 
+namespace {
+constexpr size_t MIB = (size_t)1 << 20;
+
+size_t whole_mib(size_t bytes) { return (bytes + MIB - 1) / MIB * MIB; }
+
+/* the size a block of `had` bytes grows to when `bytes` are needed: at least
+ * twice, up to WS_CAP, and a quarter more past it, so that what a stream has
+ * outgrown (kept until its release) is below twice its block up to WS_CAP, and
+ * below five times past it, however its calls grow */
+size_t grown(size_t had, size_t bytes) {
+  const size_t want = whole_mib(bytes), step = had <= WS_CAP / 2 ? 2 * had : had + had / 4;
+  const size_t least = had < WS_CAP && step > WS_CAP ? WS_CAP : step;
+  return want > least ? want : whole_mib(least);
+}
+
+/* device memory of grown() bytes, or of just what is needed where that is
+ * refused; null, with no error left, where that is too */
+void *allocate(size_t had, size_t bytes, size_t *got) {
+  void *p = nullptr;
+  *got = grown(had, bytes);
+  if (hipMalloc(&p, *got) == hipSuccess) return p;
+  (void)hipGetLastError();
+  if (*got == whole_mib(bytes)) return nullptr;
+  *got = whole_mib(bytes);
+  if (hipMalloc(&p, *got) == hipSuccess) return p;
+  (void)hipGetLastError();
+  return nullptr;
+}
+
+/* p becomes the stream's block */
+void *take_block(const Key &key, Block &b, void *p, size_t bytes) {
+  if (b.ptr) g_retired[key].push_back(b.ptr);
+  b.ptr = p;
+  b.bytes = bytes;
+  return p;
+}
+}  // namespace
+
 void *stream_workspace(hipStream_t s, size_t bytes) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return nullptr;
@@ -81,24 +124,24 @@ void *stream_workspace(hipStream_t s, size_t bytes) {
   const Key key = stream_key(dev, s);
   Block &b = g_ws[key];
   if (b.bytes >= bytes) return b.ptr;
-  const size_t want = (bytes + (1u << 20) - 1) & ~(size_t)((1u << 20) - 1); /* whole MiB */
-  void *p = nullptr;
-  if (hipMalloc(&p, want) != hipSuccess) return nullptr;
+  size_t want = 0;
+  void *p = allocate(b.bytes, bytes, &want);
+  if (!p) return nullptr;
   if (hipMemset(p, 0, want) != hipSuccess) {
     (void)hipFree(p);
     return nullptr;
   }
-  if (b.ptr) g_retired[key].push_back(b.ptr);
-  b.ptr = p;
-  b.bytes = want;
-  return p;
+  return take_block(key, b, p, want);
 }
 
 /* stream_workspace for a route that another kernel can take without one: none
  * while the stream is being captured (a graph may be replayed beside other
  * calls on the stream, or outlive the block), and no allocation that another
- * stream's capture forbids (the block is cleared by a kernel on `s`) */
-void *stream_workspace_optional(hipStream_t s, size_t bytes) {
+ * stream's capture forbids (the block is cleared by a kernel on `s`).  Where
+ * memory is refused, the block there is, and the next DENIED_CALLS requests
+ * past it do not ask again. */
+void *stream_workspace_optional(hipStream_t s, size_t bytes, size_t *got) {
+  *got = 0;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return nullptr;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -109,22 +152,23 @@ void *stream_workspace_optional(hipStream_t s, size_t bytes) {
   std::lock_guard<std::mutex> lock(g_ws_mutex);
   const Key key = stream_key(dev, s);
   Block &b = g_ws[key];
-  if (b.bytes >= bytes) return b.ptr;
-  const size_t want = (bytes + (1u << 20) - 1) & ~(size_t)((1u << 20) - 1); /* whole MiB */
-  void *p = nullptr;
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  (void)hipThreadExchangeStreamCaptureMode(&mode);
-  const hipError_t rc = hipMalloc(&p, want);
-  (void)hipThreadExchangeStreamCaptureMode(&mode);
-  if (rc != hipSuccess) {
-    (void)hipGetLastError();
-    return nullptr;
+  if (b.bytes < bytes && b.denied == 0) {
+    size_t want = 0;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    void *p = allocate(b.bytes, bytes, &want);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (p) {
+      launch_zero_fill((uint32_t *)p, want / 4, s);
+      (void)take_block(key, b, p, want);
+    } else {
+      b.denied = DENIED_CALLS;
+    }
+  } else if (b.bytes < bytes) {
+    b.denied--;
   }
-  launch_zero_fill((uint32_t *)p, want / 4, s);
-  if (b.ptr) g_retired[key].push_back(b.ptr);
-  b.ptr = p;
-  b.bytes = want;
-  return p;
+  *got = b.bytes;
+  return b.ptr;
 }
 
 int release_stream_workspace(hipStream_t s) {
@@ -260,8 +304,8 @@ int sample_routed(const d3s::SampleArgs &a, d3s::Dtype dt, hipStream_t s, Ws w) 
   const size_t off = d3s::split_counter_bytes();
   if (const size_t want = optional_workspace_bytes(a, dt, false)) {
     if (!w.ptr && w.lazy) {
-      w.ptr = d3s::stream_workspace_optional(s, want);
-      w.bytes = w.ptr ? want : 0;
+      w.ptr = d3s::stream_workspace_optional(s, want, &w.bytes);
+      if (w.bytes > want) w.bytes = want;
     }
     if (w.ptr && w.bytes > off) {
       void *p = (char *)w.ptr + off;
@@ -272,11 +316,12 @@ int sample_routed(const d3s::SampleArgs &a, d3s::Dtype dt, hipStream_t s, Ws w) 
     }
   }
   if (a.k > d3s::generic_max_k()) { /* the sorting kernels, their keys after the counters' block */
-    if (!w.ptr && w.lazy) {
-      const size_t need = routed_workspace_bytes(a, dt);
-      w.ptr = d3s::stream_workspace(s, need);
-      if (!w.ptr) return D3S_ERR_NOMEM;
-      w.bytes = need;
+    const size_t need = routed_workspace_bytes(a, dt);
+    if (w.lazy && w.bytes < need) {
+      if (void *p = d3s::stream_workspace(s, need)) {
+        w.ptr = p;
+        w.bytes = need;
+      }
     }
     if (!w.ptr || w.bytes < off + d3s::bigk_row_bytes(a)) return w.short_rc;
     if (!d3s::launch_bigk(a, dt, (char *)w.ptr + off, w.bytes - off, s)) return w.short_rc;

@@ -100,8 +100,10 @@ void launch_ras_select(const RasArgs &r, const int32_t *first, const int32_t *re
  * outgrows is kept (a call on another thread may still be enqueueing on it)
  * until release_stream_workspace.  Null when the allocation fails. */
 void *stream_workspace(hipStream_t s, size_t bytes);
-/* The same for a route that can do without: null while `s` is being captured. */
-void *stream_workspace_optional(hipStream_t s, size_t bytes);
+/* The same for a route that can do without or with less: *got is the block's
+ * size, which is below `bytes` where memory is refused; null while `s` is being
+ * captured. */
+void *stream_workspace_optional(hipStream_t s, size_t bytes, size_t *got);
 /* Waits for the stream, then frees its block and the blocks it outgrew. */
 int release_stream_workspace(hipStream_t s);
 /* Launch the head's gemv: up to two rows by k_linear, more by launch_linear_rows. */

@@ -1,6 +1,7 @@
 """The blocks the library keeps for streams: whose they are and how much they
 hold, read from the device's free memory."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -119,3 +120,40 @@ def test_per_thread_stream_calls_beside_each_other(gpu, oracle):
     for t in threads:
         t.join()
     assert not errors, errors
+
+
+@pytest.mark.parametrize("V,k,want_probs", [(32768, 100, False), (20011, 20011, False), (20011, 6000, True)])
+def test_growing_calls_keep_little(gpu, V, k, want_probs):
+    """a batch that grows a row at a time: the stream's block and the blocks it
+    has outgrown, which stay until its release, hold a few times the last call's
+    need (the sum of every call's need is over thirty times that)"""
+    import hiprt
+    N = 64
+    need = gpu.workspace_bytes(gpu.DTYPE_F32, N, V, k)
+    bx = hiprt.to_device(np.random.default_rng(5).standard_normal((N, V)).astype(np.float32))
+    bu, ids = hiprt.to_device(np.random.default_rng(6).random((N, k), np.float32)), hiprt.DeviceBuffer(4 * N)
+    probs, cand = hiprt.DeviceBuffer(4 * N * k), hiprt.DeviceBuffer(4 * N * k)
+    s = hiprt.Stream()
+
+    def call(n):
+        assert gpu.sample_raw(bx.ptr, gpu.DTYPE_F32, n, V, V, bu.ptr, k, 1.0, 0.9, None, ids.ptr,
+                              probs.ptr if want_probs else None, cand.ptr if want_probs else None, stream=s.ptr) == 0
+
+    call(N)  # what the runtime itself takes with a stream's first launches
+    assert gpu.lib().d3s_stream_workspace_release(s.ptr) == 0
+    hiprt.synchronize()
+    time.sleep(0.5)  # (freed memory shows in the count a little later)
+    free = hiprt.free_memory()
+    for n in range(1, N + 1):
+        call(n)
+    s.synchronize()
+    held = free - hiprt.free_memory()
+    assert gpu.lib().d3s_stream_workspace_release(s.ptr) == 0
+    for _ in range(50):
+        back = free - hiprt.free_memory()
+        if back < 0.5 * need:
+            break
+        time.sleep(0.1)
+    s.destroy()
+    assert 0.5 * need < held < 4.5 * need + (8 << 20), (held, need)
+    assert back < 0.5 * need + (4 << 20), (back, need)
