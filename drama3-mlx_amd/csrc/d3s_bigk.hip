@@ -673,6 +673,9 @@ bool launch_bigk(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hipSt
         chunk = c;
       }
     }
+  /* (k the streaming kernel takes: a round of few rows takes 53 us) */
+  if (a.k <= generic_max_k() && !rounds_pay(a, (a.n_rows + chunk - 1) / chunk, 55.0, 6e-6, generic_us(a, dt)))
+    return false;
   const int64_t vstride = front ? F.vstride : bigk_vstride(a.vocab);
   for (int64_t r0 = 0; r0 < a.n_rows; r0 += chunk) {
     const int64_t n = a.n_rows - r0 < chunk ? a.n_rows - r0 : chunk;

@@ -159,12 +159,15 @@ size_t topp_workspace_bytes(const SampleArgs &a);
  * than the nucleus kernel takes): each row cut into segments, the elements
  * that can rank below k gathered in ws and ranked by one workgroup.  Rows go
  * in launches of as many as ws holds; sel_workspace_bytes is for all of them
- * (up to 256 MiB) or for one row.  Returns false when the call does not fit. */
+ * (up to 256 MiB) or for one row.  Returns false when the call does not fit, or
+ * takes so many launches for want of workspace that the streaming kernel is
+ * faster. */
 bool launch_select(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hipStream_t s);
 bool sel_takes(const SampleArgs &a);
 size_t sel_workspace_bytes(const SampleArgs &a, Dtype dt, bool one_row);
 /* Launch the wide nucleus kernels (ids only, op graph's order, k > 4096, rows
- * longer than the nucleus kernel takes): no sort.  Workspace as launch_select's. */
+ * longer than the nucleus kernel takes): no sort.  Workspace, and the calls left
+ * to the kernels that take them without, as launch_select's. */
 bool launch_nucleus(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hipStream_t s);
 bool nucleus_takes(const SampleArgs &a);
 size_t nucleus_workspace_bytes(const SampleArgs &a, Dtype dt, bool one_row);
@@ -175,7 +178,8 @@ int generic_max_k();
  * k <= V): each row cut into up to 16 segments, its keys radix-sorted in ws
  * and the tail taken over the segments (bigk_row_bytes per row: keys, count
  * tables, records, tile sums; rows go in launches of as many as ws holds).
- * Returns false when ws does not hold one row. */
+ * Returns false when ws does not hold one row (or, for k the streaming kernel
+ * takes, so few that it is faster). */
 bool launch_bigk(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hipStream_t s);
 size_t bigk_row_bytes(const SampleArgs &a);
 /* the workspace with which every row (or as many as `cap` holds) goes in one

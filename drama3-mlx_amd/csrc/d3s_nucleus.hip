@@ -24,6 +24,8 @@
  * bf16, N(0, 3) logits, top_p 0.9: 5.3 + 15.5 + 8.9 + 10.0 + 12.4 + 12.3 us (62 us
  * a call) against 175 us for the sorting kernels; N(0, 0.3) logits (93% of the
  * ranks kept) 149 against 182 us; one row 43 against 105 us. */
+#include <algorithm>
+
 #include "d3s_select.h"
 
 #pragma clang fp contract(off)
@@ -854,6 +856,17 @@ bool launch_nucleus(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hi
     sel_front_shape(F, a, dt, chunk);
     if (nuc_row_bytes(F) * (size_t)chunk <= ws_bytes) break;
     if (chunk == 1) return false;
+  }
+  /* against the streaming kernel, or beyond its k the sorting kernels in the same
+   * memory (a round of one row: 39 us at V = 20 000, 98 us at 151 936; 64 rows
+   * there 167 us).  Here a round of one row takes 34 and 42 us, 64 rows 60 us. */
+  const int64_t groups = (a.n_rows + chunk - 1) / chunk;
+  if (a.k <= generic_max_k()) {
+    if (!rounds_pay(a, groups, 45.0, 6e-6, generic_us(a, dt))) return false;
+  } else {
+    const int64_t sorted = std::max<int64_t>(1, (int64_t)(ws_bytes / bigk_row_bytes(a)));
+    const double sort_us = (double)((a.n_rows + sorted - 1) / sorted) * (30.0 + 4.5e-4 * a.vocab);
+    if (!rounds_pay(a, groups, 45.0, -3e-6, sort_us)) return false; /* (4 against 7 ps an element) */
   }
   for (int64_t r0 = 0; r0 < a.n_rows; r0 += chunk) {
     const int64_t n = a.n_rows - r0 < chunk ? a.n_rows - r0 : chunk;

@@ -265,6 +265,16 @@ inline SampleArgs rows_from(const SampleArgs &a, Dtype dt, int64_t r0, int64_t n
   return c;
 }
 
+/* Whether rows taken in `groups` rounds of launches, for want of workspace, are
+ * worth it against one launch of the streaming kernel: a round's latency
+ * (group_us) and the elements' work (element_us) against generic_us.  One round
+ * always is.  [1024, 20000] bf16, k = 100: 512 rounds of two rows took 20.4 ms, 64
+ * of 16 rows 1.36 ms, the streaming kernel 0.19 ms, one round 0.076 ms. */
+double generic_us(const SampleArgs &a, Dtype dt);
+inline bool rounds_pay(const SampleArgs &a, int64_t groups, double group_us, double element_us, double other_us) {
+  return groups <= 1 || (double)groups * group_us + element_us * (double)a.n_rows * (double)a.vocab <= other_us;
+}
+
 /* The selecting kernels as a front: with L, the sorting path's (k < V: only the
  * elements that can rank below k, as keys in L; fills its records and counts);
  * without, the wide nucleus path's (each segment's counts and exact sums per

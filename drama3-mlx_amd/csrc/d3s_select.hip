@@ -549,6 +549,16 @@ size_t sel_workspace_bytes(const SampleArgs &a, Dtype dt, bool one_row) {
   return all;
 }
 
+/* The streaming kernel's time by its measured rows: one row's passes and sort
+ * (bf16, k = 100: 37 us at V = 8193, 70 us at 20 000, 436 us at 151 936; fp32
+ * a quarter less), and from about 400 rows on their number (1024 rows: 97, 192
+ * and 1375 us).  Rather too little than too much. */
+double generic_us(const SampleArgs &a, Dtype dt) {
+  const double row = 14.0 + (dt == DT_F32 ? 2.0e-3 : 2.7e-3) * a.vocab + 0.01 * a.k;
+  const double rounds = 0.62 / 256.0 * a.n_rows;
+  return row * (rounds > 1.0 ? rounds : 1.0);
+}
+
 bool launch_select(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hipStream_t s) {
   if (!ws || !sel_takes(a)) return false;
   /* the rows of a launch: as many as ws holds, each launch's rows cut into the
@@ -560,6 +570,8 @@ bool launch_select(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hip
     if (sel_row_bytes(a, L.nseg) * (size_t)chunk <= ws_bytes) break;
     if (chunk == 1) return false;
   }
+  /* (a round of few rows takes 20 to 24 us at any V; 2.7 to 4.5 ps an element) */
+  if (!rounds_pay(a, (a.n_rows + chunk - 1) / chunk, 22.0, 4.5e-6, generic_us(a, dt))) return false;
   for (int64_t r0 = 0; r0 < a.n_rows; r0 += chunk) {
     const int64_t n = a.n_rows - r0 < chunk ? a.n_rows - r0 : chunk;
     const SampleArgs c = rows_from(a, dt, r0, n);
