@@ -165,6 +165,27 @@ __device__ __forceinline__ void generic_tail_opgraph(const SampleArgs &a, const 
   }
 }
 
+/* The n (a power of two) keys of list (LDS) sorted, descending, by the
+ * BLOCK-thread workgroup; ends with a barrier (the caller's before it). */
+template <int BLOCK>
+__device__ __forceinline__ void bitonic_sort(uint64_t *list, const int n) {
+  for (int size = 2; size <= n; size <<= 1) {
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      for (int i = (int)threadIdx.x; i < n / 2; i += BLOCK) {
+        const int lo = 2 * i - (i & (stride - 1));
+        const int hi = lo + stride;
+        const uint64_t A = list[lo], B = list[hi];
+        const bool desc = (lo & size) == 0;
+        if (desc ? (A < B) : (A > B)) {
+          list[lo] = B;
+          list[hi] = A;
+        }
+      }
+      __syncthreads();
+    }
+  }
+}
+
 /* Row `row` by the whole BLOCK-thread workgroup (BLOCK a multiple of 256);
  * glist: LDS for kpow >= k composite keys (kpow a power of two); src(i): the
  * row's logit i as fp32, -inf at the banned index.  Every thread of the
@@ -283,22 +304,7 @@ __device__ __forceinline__ void generic_row_src(const SampleArgs &a, const int r
   __syncthreads();
   for (int i = k + tid; i < kpow; i += GBLOCK) glist[i] = 0ull; /* sorts last */
   __syncthreads();
-  /* ---- bitonic sort, descending */
-  for (int size = 2; size <= kpow; size <<= 1) {
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int i = tid; i < kpow / 2; i += GBLOCK) {
-        const int lo = 2 * i - (i & (stride - 1));
-        const int hi = lo + stride;
-        const uint64_t A = glist[lo], B = glist[hi];
-        const bool desc = (lo & size) == 0;
-        if (desc ? (A < B) : (A > B)) {
-          glist[lo] = B;
-          glist[hi] = A;
-        }
-      }
-      __syncthreads();
-    }
-  }
+  bitonic_sort<BLOCK>(glist, kpow);
 
   const float top_p = rp.top_p;
   if (!a.opgraph) { /* the reference kernel's order (k <= 64 then) */

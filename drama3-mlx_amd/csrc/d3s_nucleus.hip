@@ -172,10 +172,12 @@ __global__ __launch_bounds__(NU_T) void k_nuc_bound(SampleArgs a, SelLayout F, N
   uint64_t S;
   const uint32_t r0 = block_excl_scan_u32<NU_NW>(c[0] + c[1], sh, n_all);
   const uint64_t p0 = nuc_scan(q[0] + q[1], sq, S);
+  /* (the last bucket's count is what the others leave of the row) */
+  if (tid == NU_T - 1) c[1] = (uint32_t)a.vocab - n_all;
   start[2 * tid] = r0;
   start[2 * tid + 1] = r0 + c[0];
   ((uint2 *)(N.start + (size_t)row * SEL_NB))[tid] = make_uint2(r0, r0 + c[0]);
-  if (tid == 0) start[SEL_NB] = n_all;
+  if (tid == 0) start[SEL_NB] = (uint32_t)a.vocab;
   const float lse = M + d3s_logf(d3s_fixsum_to_f32(S));
   const uint32_t k = (uint32_t)a.k;
 

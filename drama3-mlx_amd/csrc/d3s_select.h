@@ -15,6 +15,8 @@ constexpr int SEL_WGS = 512;         /* workgroups a launch aims at: two per CU 
 constexpr int SEL_NB = 2048;         /* buckets below a row's max */
 constexpr float SEL_SCALE = 64.0f;   /* buckets per unit of x: 32 units, where the terms of the
                                         exact sum end (e^-28 < 2^-40) */
+constexpr float SEL_NEAR = 8.0f;     /* the selection's buckets: this, plus the distance, by its */
+constexpr int SEL_OCT_LOG2 = 8;      /* exponent and 8 mantissa bits: 8 octaves of 256 */
 constexpr int SEL_G = 32;            /* buckets a group */
 constexpr int SEL_NG = SEL_NB / SEL_G;
 constexpr int SEL_MAX_K = 4096;      /* largest k k_sel_sort takes */
@@ -27,12 +29,14 @@ struct SelSeg {
   float lmax;     /* the segment's largest logit (NaN propagates) */
   uint32_t count; /* its keys gathered */
   uint32_t masked; /* some logit is -inf (asked for at T = +inf only) */
+  uint32_t crowd;  /* the row's bucket (+ 1) whose elements are not gathered, being too many; else 0 */
+  float least;     /* what the row's gathered logits reach */
   uint64_t sum;   /* its exact sum of fix40(d3s_expf(x - m)) */
 };
 
 struct SelLayout {
   uint64_t *keys;  /* [n][vstride]: segment s's at s segc EPC: (logit bits, index) */
-  uint32_t *cnt;   /* [n][nseg][SEL_NB]: the segment's elements of each bucket */
+  uint32_t *cnt;   /* [n][nseg][SEL_NB]: the segment's elements of each bucket (0 for the last) */
   uint32_t *group; /* [n][nseg][SEL_NG]: and of each group of buckets */
   uint64_t *csum;  /* [n][nseg][SEL_NB]: the buckets' exact sums (for the wide nucleus path) */
   SelSeg *seg;     /* [n][SEL_SMAX] */
@@ -237,15 +241,68 @@ __device__ __forceinline__ bool sel_t_easy(float T) {
 /* the bucket of z = x - m <= 0 (-inf: the last) */
 __device__ __forceinline__ int sel_bucket(float z) { return (int)fminf(z * -SEL_SCALE, (float)(SEL_NB - 1)); }
 
-/* a bound every logit of the buckets up to b reaches: (b + 1) / SEL_SCALE below
- * m, with room for the roundings of x, of x - m and of this bound */
-__device__ __forceinline__ float sel_logit_bound(float M, float T, int b) {
+/* a bound every logit of x >= xc - (the roundings of x, of x - m and of this
+ * bound) reaches */
+__device__ __forceinline__ float sel_logit_from(float M, float T, float xc) {
   const float ninf = -__builtin_inff();
-  if (b >= SEL_NB - 1 || !(T < __builtin_inff())) return ninf;
-  const float xc = M - ((float)(b + 1) * (1.0f / SEL_SCALE)) * 1.0001f;
   float Lc = (xc - (fabsf(M) + fabsf(xc) + 1.0f) * 0x1p-20f) * T;
   Lc = Lc - fabsf(Lc) * 0x1p-20f;
   return Lc >= -0x1.fffffep127f ? Lc : ninf;
+}
+
+/* a bound every logit of the buckets up to b reaches: (b + 1) / SEL_SCALE below
+ * m */
+__device__ __forceinline__ float sel_logit_bound(float M, float T, int b) {
+  if (b >= SEL_NB - 1 || !(T < __builtin_inff())) return -__builtin_inff();
+  return sel_logit_from(M, T, M - ((float)(b + 1) * (1.0f / SEL_SCALE)) * 1.0001f);
+}
+
+/* The selection's buckets, of z times s = sel_rank_scale(T): what they divide
+ * is a row's logits, since the k-th of a model's logits lies at some 8 to 15
+ * units of L below the first at any T (x = L / T: 0.5 to 1.5 million at the
+ * smallest T, where buckets of x held nearly all of a row in the last).  1/32
+ * wide in the first 8 units, 1/16 to 24, and so on to 2040 units: rows of other
+ * scales keep a relative width of 1/256.  (Equal widths and then 32 an octave,
+ * four instructions an element more: 540 us against 490 us at [256, 700001].) */
+__device__ __forceinline__ float sel_rank_scale(float T) { return fminf(T, 1.0f); }
+
+/* z <= 0 */
+__device__ __forceinline__ int sel_rank_bucket(float z, float s) {
+  constexpr uint32_t near = __builtin_bit_cast(uint32_t, SEL_NEAR) >> (23 - SEL_OCT_LOG2);
+  const uint32_t t = d3s_f2u(__builtin_fmaf(z, -s, SEL_NEAR)) >> (23 - SEL_OCT_LOG2);
+  return (int)(min(t, near + (uint32_t)SEL_NB - 1u) - near);
+}
+
+/* the distance (times s) at which bucket b ends */
+__device__ __forceinline__ float sel_rank_end(int b) {
+  return d3s_u2f((uint32_t)(b + 1 + (int)(__builtin_bit_cast(uint32_t, SEL_NEAR) >> (23 - SEL_OCT_LOG2)))
+                 << (23 - SEL_OCT_LOG2)) - SEL_NEAR;
+}
+
+/* sel_logit_bound for them (y = 1 / T) */
+__device__ __forceinline__ float sel_rank_bound(float M, float T, float y, int b) {
+  if (b >= SEL_NB - 1 || !(T < __builtin_inff())) return -__builtin_inff();
+  return sel_logit_from(M, T, M - sel_rank_end(b) * fmaxf(y, 1.0f) * 1.0001f);
+}
+
+/* the least logit of the buckets up to b (+inf: none), over the order keys, 64
+ * of them at a time: x, x - m and its bucket are monotone in the logit.  Every
+ * lane of the wave calls it. */
+__device__ __forceinline__ float sel_rank_least(float M, float T, float y, float s, int b) {
+  uint32_t lo = d3s_ordkey(-__builtin_inff()), hi = d3s_ordkey(__builtin_inff()); /* lo: not; hi: is */
+#pragma unroll 1
+  while (hi - lo > 1u) {
+    const uint32_t step = (hi - lo + 63u) / 64u, at = min(hi, lo + (uint32_t)lane_id() * step);
+    const float x = scale_logit(d3s_from_ordkey(at), T, y, T < __builtin_inff());
+    /* (past the row's max: in the first bucket) */
+    const bool is = at == hi || (at > lo && sel_rank_bucket(fminf(x - M, 0.0f), s) <= b);
+    const uint64_t m = __ballot(is);
+    const int l = m ? (int)__builtin_ctzll(m) : WAVE; /* (lane 0 is at lo) */
+    const uint32_t first = l < WAVE ? min(hi, lo + (uint32_t)l * step) : hi;
+    lo = lo + (uint32_t)(l - 1) * step;
+    hi = first;
+  }
+  return d3s_from_ordkey(hi);
 }
 
 }  // namespace

@@ -6,8 +6,10 @@
  * chip, and read three times (once from HBM, then from the caches):
  *  k_sel_max: each segment's largest logit (so m = max x, division being
  *     monotone);
- *  k_sel_hist: every x = L / T exactly and its bucket below the max (width
- *     1 / SEL_SCALE, the last one open), counted in LDS and stored per segment
+ *  k_sel_hist: every x = L / T exactly and its bucket below the max
+ *     (sel_rank_bucket: of a logit's distance, or its relative width; for the
+ *     wide nucleus path 1/64 of x, the last one open), counted in LDS and stored
+ *     per segment
  *     (adding the segments' counts to one table by global atomics took 6.6 us
  *     more, at [32, 151936]); the segment's exact sum of fix40(d3s_expf(x - m));
  *  k_sel_gather: the first bucket at which the row's count reaches k, by groups
@@ -16,9 +18,11 @@
  *  k_sel_sort (a workgroup per row): those logits as composite keys, into LDS
  *     by bucket, each key's rank from the larger keys of its own bucket, then
  *     the op graph's tail with lse from the segments' sums.
- * A row with more gathered keys than LDS holds (crowded ties at the k-th
- * element) is sampled by the generic procedure in k_sel_sort's workgroup.
- * The sorting path (d3s_bigk.hip) takes the first three as its front.  Every result is the oracle's bits.
+ * Where the k-th element's bucket holds more than LDS does (masked logits, equal
+ * rows: ties by the thousand), it is left out of the gathered keys and
+ * k_sel_sort's workgroup finds its first elements in the row (sel_crowd).
+ * The sorting path (d3s_bigk.hip) takes the first three as its front.  Every
+ * result is the oracle's bits.
  *
  * Bound: latency (four launches; k_sel_sort is one workgroup's chain).
  * [32, 151936] bf16, k = 1000: 3.6 + 10.5 + 8.1 + 13.1 us against 438 us for
@@ -103,6 +107,7 @@ __global__ __launch_bounds__(SEL_T) void k_sel_hist(SampleArgs a, SelLayout L) {
   if (sel_row_max(L, row, T, M) != SEL_LIVE) return;
   __syncthreads();
   const bool te = sel_t_easy(T);
+  const float s = sel_rank_scale(T);
   uint64_t acc = 0ull;
   sel_chunks<BF16>(run, a.vocab, rp.banned, first, [&](const auto &v, int, uint32_t ok) {
     constexpr int EPC = BF16 ? 8 : 4;
@@ -111,15 +116,16 @@ __global__ __launch_bounds__(SEL_T) void k_sel_hist(SampleArgs a, SelLayout L) {
 #pragma unroll
     for (int e = 0; e < EPC; e++) {
       const float z = x[e] - M;
-      if ((ok >> e) & 1u) {
-        const int b = sel_bucket(z);
-        const uint64_t f = d3s_fix40_exp(z);
+      const int b = SUMS ? sel_bucket(z) : sel_rank_bucket(z, s);
+      const bool in = (ok >> e) & 1u;
+      /* (the last bucket, where a row's masked or far elements all lie, has no
+       * terms, and its count, kept as 0, is what the others leave of the row: no
+       * atomics on one word) */
+      if (in && b < SEL_NB - 1) {
         atomicAdd(&cnt[b], 1u);
-        if (SUMS)
-          atomicAdd((unsigned long long *)&bsum[b], (unsigned long long)f);
-        else
-          acc += f;
+        if (SUMS) atomicAdd((unsigned long long *)&bsum[b], (unsigned long long)d3s_fix40_exp(z));
       }
+      if (!SUMS && in) acc += d3s_fix40_exp(z);
     }
   });
   const size_t at = (size_t)row * L.nseg + seg;
@@ -216,9 +222,25 @@ __global__ __launch_bounds__(SEL_T) void k_sel_gather(SampleArgs a, SelLayout L,
   __syncthreads();
   const uint32_t fin = before + wave_scan_add_u32(lane < SEL_G ? fine[lane] : 0u);
   const int tb = tg * SEL_G + (int)__builtin_ctzll(__ballot(fin >= k) | (1ull << (SEL_G - 1)));
-  /* (a few elements below bucket tb may reach Lc as well: the set holds every
-   * element above any of its own, which is all that the ranking asks) */
-  const float Lc = sel_logit_bound(M, T, tb);
+  /* (a few elements below bucket tb may reach Lc as well, none below Lc's own
+   * bucket: the set holds every element above any of its own, which is all that
+   * the ranking asks.  Where it may be more than k_sel_sort ranks, the buckets up
+   * to tb exactly; where bucket tb alone makes it so, without that one) */
+  const float s = sel_rank_scale(T);
+  float Lc = sel_rank_bound(M, T, y, tb);
+  bool crowd = false;
+  if (!SORT) {
+    const int at_b = tb - tg * SEL_G;
+    const uint32_t next =
+        at_b + 1 < SEL_G ? readlane_u(fin, min(at_b + 1, SEL_G - 1)) : readlane_u(gin, min(tg + 1, WAVE - 1));
+    const float xc = Lc * y; /* (a little below Lc / T) */
+    const int reach = sel_rank_bucket(fminf(xc - fabsf(xc) * 0x1p-20f - M, 0.0f), s);
+    /* (uniform; the last bucket's elements are not in the counts) */
+    if (__builtin_expect(next > (uint32_t)SEL_CAP || reach > tb + 1 || tb + 2 >= SEL_NB, 0)) {
+      crowd = tb == SEL_NB - 1 || readlane_u(fin, at_b) > (uint32_t)SEL_CAP;
+      Lc = sel_rank_least(M, T, y, s, crowd ? tb - 1 : tb);
+    }
+  }
   auto pick = [&](const auto &v, uint32_t ok) -> uint32_t {
     uint32_t m = 0u;
 #pragma unroll
@@ -238,7 +260,12 @@ __global__ __launch_bounds__(SEL_T) void k_sel_gather(SampleArgs a, SelLayout L,
     tot += wn[w];
   }
   if (!SORT) {
-    if (tid == 0) L.seg[(size_t)row * SEL_SMAX + seg].count = tot;
+    if (tid == 0) {
+      SelSeg &sg = L.seg[(size_t)row * SEL_SMAX + seg];
+      sg.count = tot;
+      sg.crowd = crowd ? (uint32_t)tb + 1u : 0u;
+      sg.least = Lc;
+    }
     if (n == 0u) return;
   }
   uint64_t *out = SORT ? B.keys + (size_t)row * 2 * (size_t)B.vstride + (size_t)seg * B.rstride
@@ -389,6 +416,136 @@ __device__ __forceinline__ void sel_tail(const SampleArgs &a, int row, float lse
   }
 }
 
+struct CrowdLds {
+  uint32_t lo, hi, n, bin, above, count;
+};
+
+/* ranked[n .. k): the rest of the first k, from bucket tb, whose elements are
+ * not gathered: the row read again by the whole workgroup, in whole chunks, for
+ * the range of the bucket's order keys, for their counts by 11 bits of it until
+ * the last rank's is met (one range where all are equal, as masked logits are),
+ * and for those above; the equal ones in index order.  Bound: one CU's reads of
+ * the row (a 16-byte load a lane) and its scaling: [32, 151936] bf16, k = 1000,
+ * all but 60 logits masked: 82 us a call, 138 us for fp32 masked by finite values
+ * (773 and 763 us when such a row began again with the generic procedure, 695 and
+ * 700 us by the streaming kernel).  list: LDS for the keys, hist: SEL_NB counts, sh: GNW words. */
+template <bool BF16>
+__device__ __forceinline__ void sel_crowd(const SampleArgs &a, int row, const RowP &rp, float M, int tb, uint32_t n,
+                                          uint64_t *ranked, uint64_t *list, uint32_t *hist, uint32_t *sh) {
+  constexpr int ES = BF16 ? 2 : 4, EPC = 16 / ES, TIE = 8; /* elements a thread looks at for equal ones */
+  __shared__ CrowdLds S;
+  const int tid = (int)threadIdx.x, wid = __builtin_amdgcn_readfirstlane(tid / WAVE), V = a.vocab;
+  const float T = rp.T, y = 1.0f / T, s = sel_rank_scale(T);
+  const bool te = sel_t_easy(T);
+  const char *rowp = (const char *)a.logits + (size_t)row * (size_t)a.row_stride * ES;
+  SelRun r;
+  r.off = (int)(((uintptr_t)rowp & 15u) / ES);
+  r.src = (const uint4 *)(rowp - r.off * ES);
+  const int nchunks = (r.off + V + EPC - 1) / EPC, wch = (nchunks + GNW - 1) / GNW;
+  r.c0 = min(nchunks, wid * wch);
+  r.c1 = min(nchunks, r.c0 + wch);
+  auto each = [&](auto &&fn) { /* the bucket's order keys and their places */
+    uint4 first[2];
+    sel_load(r, r.c0, first);
+    sel_chunks<BF16>(r, V, rp.banned, first, [&](const auto &v, int p0, uint32_t ok) {
+      float x[EPC];
+      sel_scale(v, T, y, te, x);
+#pragma unroll
+      for (int e = 0; e < EPC; e++)
+        if (((ok >> e) & 1u) && sel_rank_bucket(x[e] - M, s) == tb) fn(x[e], p0 + e);
+    });
+  };
+  if (tid == 0) {
+    S.lo = ~0u;
+    S.hi = 0u;
+    S.n = 0u;
+  }
+  __syncthreads();
+  uint32_t lo = ~0u, hi = 0u;
+  each([&](float x, int) {
+    const uint32_t o = d3s_ordkey(x);
+    lo = min(lo, o);
+    hi = max(hi, o);
+  });
+  if (lo <= hi) {
+    atomicMin(&S.lo, lo);
+    atomicMax(&S.hi, hi);
+  }
+  __syncthreads();
+  lo = S.lo;
+  hi = S.hi;
+  uint32_t need = (uint32_t)a.k - n; /* of the keys in [lo, hi] */
+#pragma unroll 1
+  while (lo < hi) {
+    const int shift = max(0, 32 - __clz((int)(hi - lo)) - 11);
+    static_assert(SEL_NB == 2048 && SEL_NB == 2 * GBLOCK, "11 bits, two counts a thread");
+    ((uint2 *)hist)[tid] = make_uint2(0u, 0u);
+    __syncthreads();
+    each([&](float x, int) {
+      const uint32_t o = d3s_ordkey(x);
+      if (o >= lo && o <= hi) atomicAdd(&hist[(hi - o) >> shift], 1u);
+    });
+    __syncthreads();
+    const uint2 c = ((const uint2 *)hist)[tid];
+    uint32_t all;
+    const uint32_t before = block_excl_scan_u32<GNW>(c.x + c.y, sh, all);
+    if (before < need && before + c.x + c.y >= need) { /* one thread's */
+      const bool second = before + c.x < need;
+      S.bin = 2u * tid + (second ? 1u : 0u);
+      S.above = before + (second ? c.x : 0u);
+      S.count = second ? c.y : c.x;
+    }
+    __syncthreads();
+    need -= S.above;
+    hi -= S.bin << shift;
+    const uint32_t span = (1u << shift) - 1u;
+    lo = hi - lo > span ? hi - span : lo;
+    if (S.count == need) { /* every key of [lo, hi]: none is left to choose */
+      hi = lo - 1u;
+      need = 0u;
+    }
+    __syncthreads();
+  }
+  /* (lo == hi: `need` of the equal keys; hi == lo - 1: none) */
+  each([&](float x, int i) {
+    if (d3s_ordkey(x) > hi) list[atomicAdd(&S.n, 1u)] = composite_key(x, i);
+  });
+  __syncthreads();
+  const int m = (int)S.n;
+  int pow2 = 2;
+  while (pow2 < m) pow2 <<= 1;
+  for (int i = m + tid; i < pow2; i += GBLOCK) list[i] = 0ull; /* sorts last */
+  __syncthreads();
+  bitonic_sort<GBLOCK>(list, pow2);
+  for (int i = tid; i < m; i += GBLOCK) ranked[n + i] = list[i];
+  uint32_t base = 0u;
+#pragma unroll 1
+  for (int t0 = 0; t0 < V && base < need; t0 += TIE * GBLOCK) {
+    const int i0 = t0 + TIE * tid;
+    uint32_t tie = 0u;
+    float tx = 0.0f;
+#pragma unroll
+    for (int e = 0; e < TIE; e++)
+      if (i0 + e < V) {
+        const float x = scale_logit(load_logit<BF16>(rowp, i0 + e, rp.banned), T, y, T < __builtin_inff());
+        if (d3s_ordkey(x) == lo) {
+          tie |= 1u << e;
+          tx = x;
+        }
+      }
+    uint32_t all;
+    uint32_t at = base + block_excl_scan_u32<GNW>((uint32_t)__popc(tie), sh, all);
+#pragma unroll
+    for (int e = 0; e < TIE; e++)
+      if ((tie >> e) & 1u) {
+        if (at < need) ranked[n + m + at] = composite_key(tx, i0 + e);
+        at++;
+      }
+    base += all;
+  }
+  __syncthreads();
+}
+
 /* NQ: k <= NQ GBLOCK */
 template <bool BF16, int NQ>
 __global__ __launch_bounds__(GBLOCK) void k_sel_sort(SampleArgs a, SelLayout L, int kpow) {
@@ -404,6 +561,8 @@ __global__ __launch_bounds__(GBLOCK) void k_sel_sort(SampleArgs a, SelLayout L, 
   const SelSeg *sg0 = L.seg + (size_t)row * SEL_SMAX;
   const uint32_t segn = lane < L.nseg ? sg0[lane].count : 0u;
   const uint64_t segs = lane < L.nseg ? sg0[lane].sum : 0ull;
+  const uint32_t crowd = sg0[0].crowd;
+  const float least = sg0[0].least;
   float u[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; q++) {
@@ -420,11 +579,13 @@ __global__ __launch_bounds__(GBLOCK) void k_sel_sort(SampleArgs a, SelLayout L, 
   }
   const uint32_t inc = wave_scan_add_u32(segn);
   const uint32_t n = readlane_u(inc, WAVE - 1);
-  if (n > (uint32_t)SEL_CAP) { /* a crowded last bucket */
-    generic_row<BF16>(a, row, kpow, dyn);
-    return;
-  }
+  if (__builtin_expect(crowd != 0u, 0)) sel_crowd<BF16>(a, row, rp, M, (int)crowd - 1, n, sorted, bk, start, sh);
   const float lse = M + d3s_logf(d3s_fixsum_to_f32(wave_sum_mod64(segs)));
+  /* the gathered keys' buckets: SEL_NB equal parts of about what they span (any
+   * factor ranks them) */
+  const float span = M - least * y;
+  const float per = span > 0.0f ? fminf((float)SEL_NB * __builtin_amdgcn_rcpf(span), 0x1p100f) : 0.0f;
+  auto place = [&](float x) { return (int)fminf((M - x) * per, (float)(SEL_NB - 1)); };
   next[tid] = 0u;
   next[tid + GBLOCK] = 0u;
   if (wid == 0) {
@@ -450,7 +611,7 @@ __global__ __launch_bounds__(GBLOCK) void k_sel_sort(SampleArgs a, SelLayout L, 
     if (tid + q * GBLOCK < n) {
       const float x = scale_logit(d3s_u2f((uint32_t)(kv[q] >> 32)), T, y, T < __builtin_inff());
       kv[q] = composite_key(x, (int)(uint32_t)kv[q]);
-      atomicAdd(&next[sel_bucket(x - M)], 1u);
+      atomicAdd(&next[place(x)], 1u);
     }
   __syncthreads();
   const uint2 c = ((const uint2 *)next)[tid];
@@ -462,13 +623,13 @@ __global__ __launch_bounds__(GBLOCK) void k_sel_sort(SampleArgs a, SelLayout L, 
   /* the keys by bucket (any order within one) */
 #pragma unroll
   for (int q = 0; q < NK; q++)
-    if (tid + q * GBLOCK < n) bk[atomicAdd(&next[sel_bucket(key_x(kv[q]) - M)], 1u)] = kv[q];
+    if (tid + q * GBLOCK < n) bk[atomicAdd(&next[place(key_x(kv[q]))], 1u)] = kv[q];
   __syncthreads();
   /* next[b] is now bucket b's end; a key's rank: its bucket's start and the
    * larger keys of the bucket */
   for (uint32_t i = tid; i < n; i += GBLOCK) {
     const uint64_t my = bk[i];
-    const int b = sel_bucket(key_x(my) - M);
+    const int b = place(key_x(my));
     const uint32_t e = next[b];
     uint32_t rank = start[b];
     for (uint32_t j = start[b]; j < e; j++) rank += bk[j] > my ? 1u : 0u;

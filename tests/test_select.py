@@ -263,3 +263,50 @@ def test_small_k_leaves_the_workspace(gpu, oracle):
     hiprt.synchronize()
     assert np.array_equal(bids.download((N,), np.int32), oracle.sample(x, u, 0.8, 0.9)["ids"])
     assert np.array_equal(ws.download(fill.shape, np.uint32), fill)
+
+
+def crowded_rows(rng, V, dtype):
+    """rows whose k-th element is one of thousands in one place, or far below
+    the first"""
+    x = rows(rng, 12, V, "f32")
+    fmin = np.float32(-3.3e38)
+    few = rng.random((12, V)) < 40.0 / V
+    x[0] = np.where(few[0], x[0], -np.inf)       # masked: nearly every rank is -inf
+    x[1] = np.where(few[1], x[1], fmin)          # by the type's lowest values (-inf after / 0.7)
+    x[2] = np.where(few[2], x[2], -1e4)
+    x[3] = np.where(rng.random(V) < 0.5, np.where(few[3], x[3], fmin), -np.inf)  # two kinds of mask
+    x[4] = np.round(x[4])
+    x[5] = np.round(x[5] / 4) * 4
+    x[6] = 1.5
+    x[6, V // 2] = 1.5 + 2.0 ** -7
+    x[7] = x[7] * 100                            # a wide scale
+    x[8] = x[8] * 1e-3 + 1000                    # the last places of a large offset
+    x[9] = np.where(few[9], 30.0, -x[9] ** 2 * 1e5)  # the rest 0 to some millions down
+    x[10] = np.where(few[10], x[10], -(np.arange(V) // 900) - 50.0)  # ties in runs, the last ones first
+    x[11] = np.round(x[11] * 2) / 2
+    x[11, ::3] = -np.inf
+    return x if dtype == "f32" else W.f32_to_bf16_bits(x)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("V,k", [(8193, 65), (8193, 4096), (30011, 1000), (61003, 4096), (151936, 1025)])
+def test_crowded_and_far(gpu, oracle, dtype, V, k):
+    """the k-th element's bucket of more elements than LDS holds, or tens to
+    millions of units below the first, at temperatures from the smallest on"""
+    rng = np.random.default_rng([V, k])
+    x = crowded_rows(rng, V, dtype)
+    u = oracle.uniform(21, V, len(x), k)
+    for T in (1.0, 0.7, 0.1, 0.0, 40.0):
+        check(gpu, oracle, x, u, T, 0.9)
+    ban = np.where(np.arange(12) % 2, 0, V - 1).astype(np.int32)
+    check(gpu, oracle, x, u, 0.3, 1.0, banned=ban)
+
+
+@pytest.mark.parametrize("T", [1e-5, 0.05, 0.3])
+def test_small_temperatures(gpu, oracle, T):
+    rng = np.random.default_rng(22)
+    for V, k, dtype in ((8193, 300, "f32"), (50021, 4096, "bf16"), (700001, 64, "bf16")):
+        check(gpu, oracle, rows(rng, 3, V, dtype), oracle.uniform(23, V, 3, k), T, 0.95)
+    # the sorting path's front
+    for k in (5000, 24000):
+        check(gpu, oracle, rows(rng, 3, 50021, "f32"), oracle.uniform(24, k, 3, k), T, 0.95)
