@@ -16,8 +16,9 @@
  *     of buckets and then within one; the logits that can lie in it or above
  *     (few more than k), each segment's in a region of its own;
  *  k_sel_sort (a workgroup per row): those logits as composite keys, into LDS
- *     by bucket, each key's rank from the larger keys of its own bucket, then
- *     the op graph's tail with lse from the segments' sums.
+ *     by bucket, each key's rank from the larger keys of its own bucket (or, with
+ *     many in one, a radix sort), then the op graph's tail with lse from the
+ *     segments' sums.
  * Where the k-th element's bucket holds more than LDS does (masked logits, equal
  * rows: ties by the thousand), it is left out of the gathered keys and
  * k_sel_sort's workgroup finds its first elements in the row (sel_crowd).
@@ -39,6 +40,13 @@ namespace d3s {
 namespace {
 
 constexpr int SEL_CAP = 8192; /* keys k_sel_sort ranks */
+/* comparisons a thread makes where keys are ranked by all pairs of a bucket (the
+ * most crowded one's keys, for each of its own); past that all go through
+ * sel_radix (rounded and quantised logits).  us a call, bf16: [512, 20000], k =
+ * 4096, whole numbers: 1043 by pairs, 100 by the radix sort; [32, 151936], k =
+ * 4096, eighths: 98 and 48.5; k = 1000, eighths, below the line: 38.5 and 41.6;
+ * [1024, 20000], k = 4096, text, below it: 139 and 157. */
+constexpr uint32_t SEL_PAIRS = 384;
 
 template <bool BF16>
 __global__ __launch_bounds__(SEL_T) void k_sel_max(SampleArgs a, SelLayout L) {
@@ -546,13 +554,92 @@ __device__ __forceinline__ void sel_crowd(const SampleArgs &a, int row, const Ro
   __syncthreads();
 }
 
+/* n composite keys, thread t holding keys t + q GBLOCK of their index order,
+ * into list in rank order: a stable radix sort by 8 bits a pass of the order
+ * keys' bits that differ (rounded logits: one pass, bf16 ones two), so equal x
+ * stay in index order.  Each wave holds a run of the keys and counts its digits
+ * alone.  tab: GNW NB words of LDS, sh: two. */
+template <int NK>
+__device__ __forceinline__ void sel_radix(const uint64_t (&kv)[NK], uint32_t n, uint64_t *list, uint32_t *tab,
+                                          uint32_t *sh) {
+  static_assert(GNW * NB == 4 * GBLOCK && NB == 4 * WAVE, "a thread clears 16 bytes; a lane sums four digits");
+  __shared__ __align__(16) uint32_t dig[NB];
+  const int tid = (int)threadIdx.x, lane = lane_id(), wid = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const uint64_t lt = (1ull << lane) - 1ull;
+  if (tid == 0) {
+    sh[0] = 0u;
+    sh[1] = ~0u;
+  }
+  __syncthreads();
+  uint32_t some = 0u, every = ~0u;
+#pragma unroll
+  for (int q = 0; q < NK; q++)
+    if (tid + q * GBLOCK < (int)n) {
+      list[tid + q * GBLOCK] = kv[q];
+      some |= (uint32_t)(kv[q] >> 32);
+      every &= (uint32_t)(kv[q] >> 32);
+    }
+  atomicOr(&sh[0], some);
+  atomicAnd(&sh[1], every);
+  __syncthreads();
+  const uint32_t differ = sh[0] & ~sh[1];
+  uint32_t *mine = tab + wid * NB;
+#pragma unroll 1
+  for (int shift = differ ? __builtin_ctz(differ) : 32; shift < 32 && (differ >> shift); shift += 8) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) tab[tid + j * GBLOCK] = 0u;
+    __syncthreads();
+    uint64_t key[NK];
+    uint32_t at[NK]; /* the key's place among its wave's of that digit */
+#pragma unroll
+    for (int q = 0; q < NK; q++) {
+      const int i = (wid * NK + q) * WAVE + lane;
+      const bool in = i < (int)n;
+      key[q] = in ? list[i] : 0ull;
+      const uint32_t d = (~(uint32_t)(key[q] >> 32) >> shift) & 255u;
+      const uint64_t peers = wave_peers<8>(d, __ballot(in));
+      const uint32_t below = (uint32_t)__popcll(peers & lt), had = mine[d];
+      wave_lds_sync();
+      if (in && below == 0u) mine[d] = had + (uint32_t)__popcll(peers);
+      wave_lds_sync();
+      at[q] = had + below;
+      __builtin_amdgcn_sched_barrier(0); /* (one key's ballots at a time: registers) */
+    }
+    __syncthreads();
+    if (tid < NB) { /* each digit's waves in turn */
+      uint32_t run = 0u;
+#pragma unroll
+      for (int w = 0; w < GNW; w++) {
+        const uint32_t c = tab[w * NB + tid];
+        tab[w * NB + tid] = run;
+        run += c;
+      }
+      dig[tid] = run;
+    }
+    __syncthreads();
+    if (wid == 0) { /* and the digits before: a lane four of them */
+      const uint4 c = ((const uint4 *)dig)[lane];
+      const uint32_t sum = c.x + c.y + c.z + c.w, before = wave_scan_add_u32(sum) - sum;
+      ((uint4 *)dig)[lane] = make_uint4(before, before + c.x, before + c.x + c.y, before + c.x + c.y + c.z);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NK; q++) {
+      const uint32_t d = (~(uint32_t)(key[q] >> 32) >> shift) & 255u;
+      if ((wid * NK + q) * WAVE + lane < (int)n) list[dig[d] + mine[d] + at[q]] = key[q];
+    }
+    __syncthreads();
+  }
+}
+
 /* NQ: k <= NQ GBLOCK */
 template <bool BF16, int NQ>
 __global__ __launch_bounds__(GBLOCK) void k_sel_sort(SampleArgs a, SelLayout L, int kpow) {
   extern __shared__ uint64_t dyn[];
   uint64_t *sorted = dyn, *bk = dyn + kpow; /* [kpow], [SEL_CAP] */
-  __shared__ uint32_t start[SEL_NB], next[SEL_NB];
-  __shared__ uint32_t sh[GNW], sbase[SEL_SMAX + 1];
+  __shared__ __align__(16) uint32_t tab[2 * SEL_NB];
+  uint32_t *start = tab, *next = tab + SEL_NB;
+  __shared__ uint32_t sh[GNW], sbase[SEL_SMAX + 1], many;
   constexpr int PER = SEL_NB / GBLOCK, EPC = BF16 ? 8 : 4, NK = SEL_CAP / GBLOCK;
   static_assert(PER == 2 && SEL_SMAX == WAVE, "");
   const int row = (int)blockIdx.x, tid = (int)threadIdx.x, lane = lane_id();
@@ -588,6 +675,7 @@ __global__ __launch_bounds__(GBLOCK) void k_sel_sort(SampleArgs a, SelLayout L, 
   auto place = [&](float x) { return (int)fminf((M - x) * per, (float)(SEL_NB - 1)); };
   next[tid] = 0u;
   next[tid + GBLOCK] = 0u;
+  if (tid == 0) many = 0u;
   if (wid == 0) {
     sbase[lane + 1] = inc;
     if (lane == 0) sbase[0] = 0u;
@@ -615,25 +703,31 @@ __global__ __launch_bounds__(GBLOCK) void k_sel_sort(SampleArgs a, SelLayout L, 
     }
   __syncthreads();
   const uint2 c = ((const uint2 *)next)[tid];
+  if (max(c.x, c.y) * ((n + GBLOCK - 1) / GBLOCK) > SEL_PAIRS) many = 1u;
   uint32_t all;
   const uint32_t before = block_excl_scan_u32<GNW>(c.x + c.y, sh, all);
-  ((uint2 *)start)[tid] = make_uint2(before, before + c.x);
-  ((uint2 *)next)[tid] = make_uint2(before, before + c.x);
-  __syncthreads();
-  /* the keys by bucket (any order within one) */
+  if (__builtin_expect(many != 0u, 0)) { /* (uniform: the scan's barriers) */
+    sel_radix<NK>(kv, n, bk, tab, sh);
+    for (int i = tid; i < min((int)n, a.k); i += GBLOCK) sorted[i] = bk[i];
+  } else {
+    ((uint2 *)start)[tid] = make_uint2(before, before + c.x);
+    ((uint2 *)next)[tid] = make_uint2(before, before + c.x);
+    __syncthreads();
+    /* the keys by bucket (any order within one) */
 #pragma unroll
-  for (int q = 0; q < NK; q++)
-    if (tid + q * GBLOCK < n) bk[atomicAdd(&next[place(key_x(kv[q]))], 1u)] = kv[q];
-  __syncthreads();
-  /* next[b] is now bucket b's end; a key's rank: its bucket's start and the
-   * larger keys of the bucket */
-  for (uint32_t i = tid; i < n; i += GBLOCK) {
-    const uint64_t my = bk[i];
-    const int b = place(key_x(my));
-    const uint32_t e = next[b];
-    uint32_t rank = start[b];
-    for (uint32_t j = start[b]; j < e; j++) rank += bk[j] > my ? 1u : 0u;
-    if (rank < (uint32_t)a.k) sorted[rank] = my;
+    for (int q = 0; q < NK; q++)
+      if (tid + q * GBLOCK < n) bk[atomicAdd(&next[place(key_x(kv[q]))], 1u)] = kv[q];
+    __syncthreads();
+    /* next[b] is now bucket b's end; a key's rank: its bucket's start and the
+     * larger keys of the bucket */
+    for (uint32_t i = tid; i < n; i += GBLOCK) {
+      const uint64_t my = bk[i];
+      const int b = place(key_x(my));
+      const uint32_t e = next[b];
+      uint32_t rank = start[b];
+      for (uint32_t j = start[b]; j < e; j++) rank += bk[j] > my ? 1u : 0u;
+      if (rank < (uint32_t)a.k) sorted[rank] = my;
+    }
   }
   __syncthreads();
   sel_tail<NQ>(a, row, lse, rp.top_p, sorted, u);

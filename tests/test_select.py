@@ -310,3 +310,19 @@ def test_small_temperatures(gpu, oracle, T):
     # the sorting path's front
     for k in (5000, 24000):
         check(gpu, oracle, rows(rng, 3, 50021, "f32"), oracle.uniform(24, k, 3, k), T, 0.95)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("N,V,k,step", [(3, 8193, 500, 1.0), (2, 20011, 4096, 1.0), (2, 40003, 4000, 0.25), (3, 9001, 1024, 4.0),
+                                        (2, 30001, 2500, 2.0 ** -7)])
+def test_quantised_logits(gpu, oracle, dtype, N, V, k, step):
+    """logits of few different values: the gathered keys crowd in k_sel_sort's
+    buckets and go through its radix sort, 1 to 4 passes of it"""
+    rng = np.random.default_rng([V, k])
+    x = (np.round(rng.standard_normal((N, V)) * 3 / step) * step).astype(np.float32)
+    x[0, :40] += 9.5
+    x[-1] -= 100.25  # below zero, the last places in use at T = 0.7
+    x = x if dtype == "f32" else W.f32_to_bf16_bits(x)
+    u = oracle.uniform(25, V, N, k)
+    for T in (1.0, 0.7):
+        check(gpu, oracle, x, u, T, 0.97)
