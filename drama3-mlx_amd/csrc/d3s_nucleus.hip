@@ -15,8 +15,9 @@
  *     of the buckets of those ranks that can reach the row's best, and the exact
  *     sum of fix40(d3s_expf(x - lse)) before the cut's;
  *  k_nuc_final (a workgroup per row): the cut and the kept sum exactly, the
- *     ranks' elements (by sorting a small gathered set, by radix descent in a
- *     large one: crowded ties, top_p near 1), their exact scores and the id.
+ *     ranks' elements (by sorting a small gathered set, by counting 11 bits of
+ *     what its keys span in a large one: crowded ties, top_p near 1), their exact
+ *     scores and the id.
  * A row whose kept ranks have no positive score (u = 0 throughout), or more
  * candidates than k_nuc_race files, is sorted by k_nuc_final's workgroup.
  *
@@ -38,9 +39,10 @@ struct NucRow {
   float M, lse;
   uint32_t state;  /* NucState */
   uint32_t b1, b2; /* the buckets the cut lies in; b1 > b2: the cut is k */
-  uint32_t n1;     /* the elements before b1, and their sum of fix40(d3s_expf(x - m)) */
+  uint32_t n1;     /* the elements before b1, and (q1) their sum of fix40(d3s_expf(x - m)) */
   uint32_t r1, r2; /* the ranks below r1 are kept, those from r2 on are not */
-  uint64_t q1;     /* (b1 > b2: the sum of all k) */
+  uint32_t open;   /* the cut is k unless it lies in b1 .. b2 (what follows adds nothing to the prefix) */
+  uint64_t q1, qk; /* qk: the sum of all k (b1 > b2, or open) */
 };
 /* a share of the ranks: the least its best kept rank can score, and the ranks
  * that can score as much, with the most they can, their buckets and the
@@ -69,8 +71,8 @@ namespace {
 
 enum NucState : uint32_t { NUC_LIVE, NUC_REFUSED, NUC_MASKED };
 constexpr int NU_T = 1024, NU_NW = NU_T / WAVE;
-constexpr uint32_t NU_SMALL = 512; /* gathered elements ranked by counting (a pass over all for each; a
-                                      descent's four to eight passes past that) */
+constexpr uint32_t NU_SMALL = 512; /* gathered elements ranked by counting (a pass over all for each; past
+                                      that a search narrows them, about three passes) */
 constexpr int NR_T = 512;          /* threads of a share's workgroup */
 constexpr uint32_t NU_TOP = 1024;  /* every share also looks at the first ranks */
 
@@ -135,7 +137,7 @@ __device__ __forceinline__ int nuc_bucket_of(const uint32_t *start, uint32_t r) 
 __global__ __launch_bounds__(NU_T) void k_nuc_bound(SampleArgs a, SelLayout F, NucLayout N) {
   __shared__ uint32_t start[SEL_NB + 1];
   __shared__ uint32_t sh[NU_NW];
-  __shared__ uint64_t sq[NU_NW], qv[2];
+  __shared__ uint64_t sq[NU_NW], qv[3];
   __shared__ int first_cut, all_drop, kth;
   const int row = (int)blockIdx.x, tid = (int)threadIdx.x;
   /* this thread's two buckets over the segments */
@@ -182,16 +184,20 @@ __global__ __launch_bounds__(NU_T) void k_nuc_bound(SampleArgs a, SelLayout F, N
   const uint32_t k = (uint32_t)a.k;
 
   /* c_r = RN(P_r 2^-40), P_r the sum of fix40(d3s_expf(x_j - lse)) over j <= r,
-   * against Q_r, the sum of fix40(d3s_expf(x_j - m)), and S = Q_V: each term of
-   * Q and S is short of its real value by less than a unit, and exp(x_j - lse)
-   * is exp(x_j - m) / sum within a factor 1 +- eps: the roundings of lse (2^-24
-   * |lse|, the log's and S's), of x_j - lse and x_j - m (2^-24 of at most 44;
-   * terms further down count nothing on either side) and two d3s_expf's
-   * (2^-22), each taken at four times its bound.  So
-   *   Q / (S + V) (1 - eps) - (r + 1) 2^-40 <= P_r 2^-40 <= (Q + r + 1) / S (1 + eps). */
-  const double tp = (double)top_p, Sd = (double)S;
-  const double eps = (double)(fabsf(lse) + 64.0f) * 0x1p-21 + 0x1p-18;
-  const bool usable = eps < 0.01;
+   * against Q_r, the sum of fix40(d3s_expf(x_j - m)): each term of either is short
+   * of its real value by less than a unit, and exp(x_j - lse) is exp(x_j - m) g,
+   * g = exp(-(lse - m)), whatever lse's own rounding (the largest part of x_j - lse
+   * for a large |lse|: T near 0).  What is left are the roundings of x_j - lse
+   * (2^-24 of at most 28: a term further down is zero), of x_j - m (28 + lse - m)
+   * and of lse - m, and three d3s_expf's (2^-23 each, counted twice), in all
+   * (68 + 2 (lse - m)) 2^-24.  So
+   *   Q g (1 - eps) - (r + 1) <= P_r <= (Q + r + 1) g (1 + eps). */
+  const float over = lse - M;
+  const double tq = (double)top_p * 0x1p40, g = (double)d3s_expf(-over);
+  const double eps = (double)(76.0f + 2.125f * over) * 0x1p-24;
+  const double g_hi = g * (1.0 + eps) * (1.0 + 0x1p-22), g_lo = g * (1.0 - eps);
+  /* the last bucket with a term of P that is not zero (x - lse > -27.73) */
+  const int bz = (int)fminf(fmaxf((27.75f - over) * SEL_SCALE + 2.0f, 0.0f), (float)(SEL_NB - 1));
   {
     uint32_t n = r0;
     uint64_t Q = p0;
@@ -201,9 +207,9 @@ __global__ __launch_bounds__(NU_T) void k_nuc_bound(SampleArgs a, SelLayout F, N
       n += c[e];
       Q += q[e];
       if (c[e]) {
-        const bool some = usable ? ((double)Q + (double)n) / Sd * (1.0 + eps) * (1.0 + 0x1p-22) > tp : tp == tp;
-        const bool all = usable && (double)Q / (Sd + (double)a.vocab) * (1.0 - eps) - ((double)n + 2.0) * 0x1p-40 >
-                                       tp + fabs(tp) * 0x1p-22;
+        const double nd = 1.001 * (double)n;
+        const bool some = ((double)Q + nd) * g_hi > tq;
+        const bool all = (double)Q * g_lo - nd - 2.0 > tq + fabs(tq) * 0x1p-22;
         if (some) vs = min(vs, 2 * tid + e); /* its last rank may be dropped */
         if (all) va = min(va, 2 * tid + e);  /* its last rank certainly is */
         if (n >= k) vk = min(vk, 2 * tid + e);
@@ -220,20 +226,25 @@ __global__ __launch_bounds__(NU_T) void k_nuc_bound(SampleArgs a, SelLayout F, N
   }
   __syncthreads();
   const int bk = kth;
-  int b1 = min(first_cut, bk);
-  const int b2 = min(all_drop, bk);
-  const bool none = first_cut > bk; /* no rank below k is dropped */
-  const bool whole = none && start[bk + 1] == k;
-  /* R1 ranks are surely kept (rank 0 always is), none past R2 is */
+  if (tid == bk / 2) {
+    qv[1] = p0 + q[0] + (bk & 1 ? q[1] : 0ull);
+    qv[2] = q[bk & 1];
+  }
+  const int fc = first_cut;
+  const bool none = fc > bk || fc > bz; /* no rank below k is dropped */
+  const int b1 = none ? bk : fc, b2 = none ? bk : min(all_drop, bk);
   if (tid == b1 / 2) qv[0] = p0 + (b1 & 1 ? q[0] : 0ull);
-  if (tid == bk / 2) qv[1] = p0 + q[0] + (bk & 1 ? q[1] : 0ull);
   __syncthreads();
+  /* all k's sum is known when they end with a bucket, or in one of zero terms;
+   * then only the buckets that can hold the cut are looked at */
+  const bool known = start[bk + 1] == k || qv[2] == 0ull;
+  const bool whole = none && known, open = !none && known && b2 > bz;
+  /* R1 ranks are surely kept (rank 0 always is), none past R2 is */
   uint32_t R1 = k;
-  const uint32_t R2 = min(k, start[b2 + 1]);
+  const uint32_t R2 = none ? k : min(k, start[b2 + 1]);
   if (!none) {
     const double step = (double)nuc_ehi(b1) * 0x1p40 + 1.0;
-    const double room = tp * Sd / ((1.0 + eps) * (1.0 + 0x1p-22)) - (double)qv[0] - (double)start[b1];
-    double j = usable ? room / step - 2.0 : 0.0;
+    double j = (tq / g_hi - (double)qv[0] - 1.001 * (double)start[b1]) / step - 2.0;
     j = j > 0.0 ? j : 0.0;
     const double most = (double)(start[b1 + 1] - start[b1]);
     R1 = start[b1] + (uint32_t)(j < most ? j : most);
@@ -246,11 +257,13 @@ __global__ __launch_bounds__(NU_T) void k_nuc_bound(SampleArgs a, SelLayout F, N
     r.lse = lse;
     r.state = NUC_LIVE;
     r.b1 = whole ? 1u : (uint32_t)b1;
-    r.b2 = whole ? 0u : (uint32_t)b2;
+    r.b2 = whole ? 0u : (uint32_t)(open ? max(bz, b1) : b2);
     r.n1 = start[b1];
     r.r1 = R1;
     r.r2 = R2;
-    r.q1 = whole ? qv[1] : qv[0];
+    r.open = open ? 1u : 0u;
+    r.q1 = qv[0];
+    r.qk = qv[1];
     *out = r;
   }
 }
@@ -503,123 +516,233 @@ struct NucSet {
 };
 
 struct NucLds {
-  uint64_t list[NU_SMALL + 2], ranked[NU_SMALL]; /* (the sort's places by wave and digit as well) */
-  uint32_t wcnt[NU_NW][NB];
-  uint64_t ps[NB], ks[NB];
-  uint32_t hist[NB];
-  uint64_t sq[NU_NW];
-  uint32_t sh[NU_NW];
+  uint64_t list[NU_SMALL + 2], ranked[NU_SMALL];
+  union {
+    struct { /* a large set's counts and sums by 11 bits of what its keys span */
+      uint64_t ps[SEL_NB], ks[SEL_NB];
+      uint32_t hist[SEL_NB];
+    };
+    struct { /* nuc_sort_row's places by wave and digit */
+      uint32_t wcnt[NU_NW][NB], base[NB];
+    };
+  };
+  uint64_t sq[NU_NW], lo, hi, p, k;
+  uint32_t sh[NU_NW], n, above, count;
+  int bin;
   uint32_t abase[BK_SMAX + 1], bbase[BK_SMAX + 1];
   uint64_t ckey[WAVE];
   uint32_t crank[WAVE], cbucket[WAVE], cstart[WAVE];
 };
 
-/* the cut and the kept sum in a large set of the cut's buckets: by 8-bit
- * digits of the order key, descending, with the exact sums of each digit's
- * elements; the last group's elements are equal.  R, P, K: the ranks and sums
- * before the set. */
-__device__ __forceinline__ void nuc_descend(const NucSet &A, NucLds &L, float M, float lse, float top_p, uint32_t k,
-                                            uint32_t R, uint64_t P, uint64_t K, uint32_t &cut, uint64_t &kept) {
-  const int lane = lane_id(), tid = (int)threadIdx.x;
-  uint32_t prefix = 0u, pmask = 0u;
-#pragma unroll 1
-  for (int shift = 24; shift >= 0; shift -= 8) {
-    __syncthreads();
-    if (tid < NB) {
-      L.hist[tid] = 0u;
-      L.ps[tid] = 0ull;
-      L.ks[tid] = 0ull;
+/* how far to shift what [0, span] holds for 11 bits of it */
+__device__ __forceinline__ int nuc_shift(uint64_t span) {
+  return span ? max(0, 64 - (int)__builtin_clzll(span) - 11) : 0;
+}
+
+/* the least and greatest val(key) of a set's keys for which in(key); lo > hi:
+ * none.  Opens and ends with a barrier. */
+template <class In, class Val>
+__device__ __forceinline__ void nuc_range(const NucSet &A, NucLds &L, uint64_t &lo, uint64_t &hi, In &&in, Val &&val) {
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    L.lo = ~0ull;
+    L.hi = 0ull;
+  }
+  __syncthreads();
+  lo = ~0ull;
+  hi = 0ull;
+  A.each([&](uint64_t key) {
+    if (in(key)) {
+      const uint64_t v = val(key);
+      lo = v < lo ? v : lo;
+      hi = v > hi ? v : hi;
     }
+  });
+  if (lo <= hi) {
+    atomicMin((unsigned long long *)&L.lo, (unsigned long long)lo);
+    atomicMax((unsigned long long *)&L.hi, (unsigned long long)hi);
+  }
+  __syncthreads();
+  lo = L.lo;
+  hi = L.hi;
+}
+
+/* the keys of a set for which in(key), at most NU_SMALL of them, ranked */
+template <class In>
+__device__ __forceinline__ uint32_t nuc_collect(const NucSet &A, NucLds &L, In &&in) {
+  __syncthreads();
+  if (threadIdx.x == 0) L.n = 0u;
+  __syncthreads();
+  A.each([&](uint64_t key) {
+    if (in(key)) L.list[atomicAdd(&L.n, 1u)] = key;
+  });
+  __syncthreads();
+  const uint32_t n = L.n;
+  rank_by_count<NU_T>(L.list, n, (int)n, L.ranked);
+  return n;
+}
+
+/* what a search for the cut has behind it: ranks, their sums of
+ * fix40(d3s_expf(x - lse)) and of fix40(d3s_expf(x - m)) */
+struct NucSum {
+  uint32_t n;
+  uint64_t p, k;
+};
+
+/* whether a rank r = at.n - 1 that ends with these sums is dropped, or is past k */
+__device__ __forceinline__ bool nuc_past(uint32_t n, uint64_t p, uint32_t k, float top_p) {
+  return n > k || (n > 1u && d3s_fixsum_to_f32(p) > top_p);
+}
+
+/* the cut among the n ranked keys of L.ranked, from `at` on; at: the ranks
+ * before the cut and their sums (all of them when it is not there) */
+__device__ __forceinline__ bool nuc_cut_small(NucLds &L, uint32_t n, float M, float lse, float top_p, uint32_t k,
+                                              NucSum &at) {
+  const int tid = (int)threadIdx.x, lane = lane_id(), wid = tid / WAVE;
+  const bool in = (uint32_t)tid < n;
+  const float x = in ? key_x(L.ranked[tid]) : 0.0f;
+  const uint64_t f = in ? d3s_fix40_exp(x - lse) : 0ull;
+  uint64_t tot;
+  const uint64_t P = at.p + nuc_scan(f, L.sq, tot) + f;
+  const uint32_t r = at.n + (uint32_t)tid;
+  const int cm = wave_min_i32(in && nuc_past(r + 1u, P, k, top_p) ? (int)r : 0x7fffffff);
+  if (lane == 0) L.sh[wid] = (uint32_t)cm;
+  __syncthreads();
+  uint32_t cut = at.n + n;
+#pragma unroll
+  for (int w = 0; w < NU_NW; w++) cut = min(cut, L.sh[w]);
+  uint64_t ks;
+  (void)nuc_scan(in && r < cut ? d3s_fix40_exp(x - M) : 0ull, L.sq, ks);
+  const bool hit = cut < at.n + n;
+  at.n = cut;
+  at.k += ks;
+  return hit;
+}
+
+/* The same in a large set of the cut's buckets: the range of its order keys;
+ * their counts and exact sums by 11 bits of it (the digits of a bucket's few
+ * values lie apart, where the key's leading bytes are all the same); the first
+ * digit whose last rank is dropped; and so on in that digit until its keys are
+ * few (ranked) or equal. */
+__device__ __forceinline__ bool nuc_cut_large(const NucSet &A, NucLds &L, float M, float lse, float top_p, uint32_t k,
+                                              NucSum &at) {
+  const int tid = (int)threadIdx.x;
+  uint64_t lo, hi;
+  nuc_range(A, L, lo, hi, [](uint64_t) { return true; }, [](uint64_t key) { return key >> 32; });
+  uint32_t count = A.n;
+#pragma unroll 1
+  while (lo < hi) {
+    if (count <= NU_SMALL) {
+      const uint32_t n = nuc_collect(A, L, [&](uint64_t key) { return (key >> 32) >= lo && (key >> 32) <= hi; });
+      return nuc_cut_small(L, n, M, lse, top_p, k, at);
+    }
+    const int shift = nuc_shift(hi - lo);
+    static_assert(SEL_NB == 2 * NU_T, "a thread two digits");
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      L.hist[tid + j * NU_T] = 0u;
+      L.ps[tid + j * NU_T] = L.ks[tid + j * NU_T] = 0ull;
+    }
+    if (tid == 0) L.bin = SEL_NB;
     __syncthreads();
     A.each([&](uint64_t key) {
-      const uint32_t o = (uint32_t)(key >> 32);
-      if ((o & pmask) == prefix) {
-        const int d = (o >> shift) & 255u;
+      const uint64_t o = key >> 32;
+      if (o >= lo && o <= hi) {
+        const int d = (int)((hi - o) >> shift);
         const float x = key_x(key);
+        const uint64_t f = d3s_fix40_exp(x - lse), e = d3s_fix40_exp(x - M);
         atomicAdd(&L.hist[d], 1u);
-        atomicAdd((unsigned long long *)&L.ps[d], (unsigned long long)d3s_fix40_exp(x - lse));
-        atomicAdd((unsigned long long *)&L.ks[d], (unsigned long long)d3s_fix40_exp(x - M));
+        if (f) atomicAdd((unsigned long long *)&L.ps[d], (unsigned long long)f);
+        if (e) atomicAdd((unsigned long long *)&L.ks[d], (unsigned long long)e);
       }
     });
     __syncthreads();
-    /* every wave alike: digits 255 - 4 lane - q, the first whose last rank is
-     * dropped, or which holds rank k */
-    uint32_t c[4], cl = 0u;
-    uint64_t p[4], pl = 0ull, kk[4], kl = 0ull;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int d = NB - 1 - 4 * lane - q;
-      c[q] = L.hist[d];
-      p[q] = L.ps[d];
-      kk[q] = L.ks[d];
-      cl += c[q];
-      pl += p[q];
-      kl += kk[q];
+    const uint32_t c0 = L.hist[2 * tid], c1 = L.hist[2 * tid + 1];
+    const uint64_t p0 = L.ps[2 * tid], p1 = L.ps[2 * tid + 1], k0 = L.ks[2 * tid], k1 = L.ks[2 * tid + 1];
+    uint32_t nt;
+    uint64_t pt, kt;
+    const uint32_t nb = at.n + block_excl_scan_u32<NU_NW>(c0 + c1, L.sh, nt);
+    const uint64_t pb = at.p + nuc_scan(p0 + p1, L.sq, pt), kb = at.k + nuc_scan(k0 + k1, L.sq, kt);
+    const bool past0 = c0 && nuc_past(nb + c0, pb + p0, k, top_p);
+    const bool past1 = c1 && nuc_past(nb + c0 + c1, pb + p0 + p1, k, top_p);
+    const int b = wave_min_i32(past0 ? 2 * tid : past1 ? 2 * tid + 1 : SEL_NB);
+    if (lane_id() == 0 && b < SEL_NB) atomicMin(&L.bin, b);
+    __syncthreads();
+    const int bin = L.bin;
+    if (bin == SEL_NB) { /* no cut in the set */
+      at.n += nt;
+      at.p += pt;
+      at.k += kt;
+      return false;
     }
-    uint32_t n = R + wave_scan_add_u32(cl) - cl;
-    uint64_t pp = P + wave_scan_mod64(pl) - pl, kq = K + wave_scan_mod64(kl) - kl;
-    const uint32_t n_end = readlane_u(n + cl, WAVE - 1);
-    const uint64_t k_end = readlane_u64(kq + kl, WAVE - 1);
-    bool hit = false;
-    int hd = 0;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      if (!hit) {
-        const uint32_t n2 = n + c[q];
-        if (c[q] && (n2 > k || (n2 > 1u && d3s_fixsum_to_f32(pp + p[q]) > top_p))) {
-          hit = true;
-          hd = NB - 1 - 4 * lane - q;
-        } else {
-          n = n2;
-          pp += p[q];
-          kq += kk[q];
-        }
-      }
+    if (tid == bin / 2) {
+      const bool second = bin & 1;
+      L.n = nb + (second ? c0 : 0u);
+      L.p = pb + (second ? p0 : 0ull);
+      L.k = kb + (second ? k0 : 0ull);
+      L.count = second ? c1 : c0;
     }
-    const uint64_t any = __ballot(hit);
-    if (any == 0ull) { /* no cut in the set */
-      cut = min(k, n_end);
-      kept = k_end;
-      return;
-    }
-    const int l = (int)__builtin_ctzll(any);
-    prefix |= readlane_u((uint32_t)hd, l) << shift;
-    pmask |= 0xffu << shift;
-    R = readlane_u(n, l);
-    P = readlane_u64(pp, l);
-    K = readlane_u64(kq, l);
+    __syncthreads();
+    at.n = L.n;
+    at.p = L.p;
+    at.k = L.k;
+    count = L.count;
+    hi -= (uint64_t)bin << shift;
+    const uint64_t span = (1ull << shift) - 1ull;
+    lo = hi - lo > span ? hi - span : lo;
   }
-  /* equal elements: the first rank j of them (not rank 0) past top_p, or rank k */
-  const float x = d3s_from_ordkey(prefix);
-  const uint64_t f = d3s_fix40_exp(x - lse), need = d3s_fixsum_gt_threshold(top_p);
+  /* `count` equal elements: the first rank j of them (not rank 0) past top_p, or rank k */
+  const float x = d3s_from_ordkey((uint32_t)hi);
+  const uint64_t f = d3s_fix40_exp(x - lse), e = d3s_fix40_exp(x - M), need = d3s_fixsum_gt_threshold(top_p);
   uint64_t j = 0ull;
-  if (P < need) j = f && need != ~0ull ? (need - P + f - 1ull) / f - 1ull : ~0ull;
-  const uint32_t t = L.hist[prefix & 255u];
-  if (j > t) j = t;
-  cut = min(k, max(R + (uint32_t)j, 1u));
-  kept = K + (uint64_t)(cut - R) * d3s_fix40_exp(x - M);
+  if (at.p < need) j = f && need != ~0ull ? (need - at.p + f - 1ull) / f - 1ull : ~0ull;
+  if (at.n == 0u && j == 0ull) j = 1ull; /* (rank 0 is kept) */
+  if (j > count) j = count;
+  if (at.n + (uint32_t)j > k) j = k - at.n;
+  at.n += (uint32_t)j;
+  at.k += j * e;
+  return j < count;
 }
 
 /* element j (descending x, then ascending index) of the set's bucket b */
 __device__ __forceinline__ uint64_t nuc_select(const NucSet &A, NucLds &L, float M, int b, uint32_t j) {
   const int tid = (int)threadIdx.x;
-  uint64_t prefix = 0ull, pmask = 0ull;
+  auto mine = [&](uint64_t key) { return sel_bucket(key_x(key) - M) == b; };
+  uint64_t lo, hi;
+  nuc_range(A, L, lo, hi, mine, [](uint64_t key) { return key; });
   uint32_t need = j + 1u;
 #pragma unroll 1
-  for (int shift = 56; shift >= 0; shift -= 8) { /* the composite key's bytes: x, then ~index */
+  while (lo < hi) { /* (no two keys are equal) */
+    const int shift = nuc_shift(hi - lo);
     __syncthreads();
-    if (tid < NB) L.hist[tid] = 0u;
+    L.hist[tid] = L.hist[tid + NU_T] = 0u;
     __syncthreads();
     A.each([&](uint64_t key) {
-      if ((key & pmask) == prefix && sel_bucket(key_x(key) - M) == b) atomicAdd(&L.hist[(key >> shift) & 255u], 1u);
+      if (key >= lo && key <= hi && mine(key)) atomicAdd(&L.hist[(hi - key) >> shift], 1u);
     });
     __syncthreads();
-    const BinSel s = wave_find_bin<false>(L.hist, need);
-    prefix |= (uint64_t)s.bin << shift;
-    pmask |= 0xffull << shift;
-    need -= s.above;
+    const uint32_t c0 = L.hist[2 * tid], c1 = L.hist[2 * tid + 1];
+    uint32_t all;
+    const uint32_t before = block_excl_scan_u32<NU_NW>(c0 + c1, L.sh, all);
+    if (before < need && before + c0 + c1 >= need) { /* one thread's */
+      const bool second = before + c0 < need;
+      L.bin = 2 * tid + (second ? 1 : 0);
+      L.above = before + (second ? c0 : 0u);
+      L.count = second ? c1 : c0;
+    }
+    __syncthreads();
+    const uint64_t top = hi - ((uint64_t)L.bin << shift), span = (1ull << shift) - 1ull;
+    const uint32_t count = L.count;
+    need -= L.above;
+    lo = top - lo > span ? top - span : lo;
+    hi = top;
+    if (count <= NU_SMALL) {
+      (void)nuc_collect(A, L, [&](uint64_t key) { return key >= lo && key <= hi && mine(key); });
+      return L.ranked[need - 1u];
+    }
   }
-  return prefix;
+  return hi;
 }
 
 /* the row sorted by one workgroup (a stable LSD radix sort by ordkey(x)
@@ -636,7 +759,7 @@ __device__ __forceinline__ void nuc_sort_row(const SampleArgs &a, int row, const
   for (int i = tid; i < V; i += NU_T)
     src[i] = composite_key(scale_logit(load_logit<BF16>(rowp, i, rp.banned), rp.T, y, rp.T < __builtin_inff()), i);
   const uint64_t lt = (1ull << lane) - 1ull;
-  uint32_t *base = L.hist;
+  uint32_t *base = L.base;
 #pragma unroll 1
   for (int pass = 0; pass < 4; pass++) {
     __syncthreads();
@@ -709,7 +832,6 @@ __global__ __launch_bounds__(NU_T) void k_nuc_final(SampleArgs a, NucLayout N) {
   const uint32_t k = (uint32_t)a.k;
   {
     const uint32_t b1 = rec->b1, b2 = rec->b2, n1 = rec->n1;
-    const uint64_t q1 = rec->q1;
     /* the row's candidates, at most one a lane (every wave files the same) */
     uint32_t ncand = 0u;
     const bool few = nuc_candidates(N, row, [&](bool in, const NucShare *p, uint32_t slot) {
@@ -750,34 +872,27 @@ __global__ __launch_bounds__(NU_T) void k_nuc_final(SampleArgs a, NucLayout N) {
 
     /* ---- the cut and the kept sum */
     uint32_t cut = k;
-    uint64_t kept = q1;
+    uint64_t kept = rec->qk;
     const bool small_a = A.n <= NU_SMALL;
-    if (b1 <= b2 && small_a) {
-      if ((uint32_t)tid < A.n) L.list[tid] = A.at((uint32_t)tid);
-      __syncthreads();
-      rank_by_count<NU_T>(L.list, A.n, (int)A.n, L.ranked);
-      const bool in = (uint32_t)tid < A.n;
-      const float x = in ? key_x(L.ranked[tid]) : 0.0f;
-      const uint64_t f = in ? d3s_fix40_exp(x - lse) : 0ull;
-      uint64_t tot;
-      const uint64_t P = P1 + nuc_scan(f, L.sq, tot) + f;
-      const uint32_t r = n1 + (uint32_t)tid;
-      const bool stop = in && (r == k || (r > 0u && d3s_fixsum_to_f32(P) > top_p));
-      const int cm = wave_min_i32(stop ? (int)r : 0x7fffffff);
-      if (lane == 0) L.sh[wid] = (uint32_t)cm;
-      __syncthreads();
-      cut = min(k, n1 + A.n);
-#pragma unroll
-      for (int w = 0; w < NU_NW; w++) cut = min(cut, L.sh[w]);
-      uint64_t ks;
-      (void)nuc_scan(in && r < cut ? d3s_fix40_exp(x - M) : 0ull, L.sq, ks);
-      kept = q1 + ks;
-    } else if (b1 <= b2) {
-      nuc_descend(A, L, M, lse, top_p, k, n1, P1, q1, cut, kept);
+    if (b1 <= b2) {
+      NucSum at{n1, P1, rec->q1};
+      bool hit;
+      if (small_a) {
+        if ((uint32_t)tid < A.n) L.list[tid] = A.at((uint32_t)tid);
+        __syncthreads();
+        rank_by_count<NU_T>(L.list, A.n, (int)A.n, L.ranked);
+        hit = nuc_cut_small(L, A.n, M, lse, top_p, k, at);
+      } else {
+        hit = nuc_cut_large(A, L, M, lse, top_p, k, at);
+      }
+      if (hit || !rec->open) {
+        cut = min(k, at.n);
+        kept = at.k;
+      }
     }
 
     /* ---- the candidates' elements */
-    if (small_a && wid == 0 && (uint32_t)lane < ncand && cr >= n1 && b1 <= b2) L.ckey[lane] = L.ranked[cr - n1];
+    if (small_a && wid == 0 && (uint32_t)lane < ncand && cr >= n1 && cr - n1 < A.n) L.ckey[lane] = L.ranked[cr - n1];
     __syncthreads();
     const bool small_b = B.n <= NU_SMALL;
     if (small_b && B.n > 0u) {
@@ -785,22 +900,23 @@ __global__ __launch_bounds__(NU_T) void k_nuc_final(SampleArgs a, NucLayout N) {
       __syncthreads();
       rank_by_count<NU_T>(L.list, B.n, (int)B.n, L.ranked);
     }
-    for (uint32_t c = 0; c < ncand; c++) { /* (uniform) */
-      const uint32_t r = readlane_u(cr, (int)c), s = readlane_u(cs, (int)c);
-      const int b = (int)readlane_u((uint32_t)cb, (int)c);
-      const bool in_a = b1 <= b2 && r >= n1;
-      if (in_a && small_a) continue;
-      if (!in_a && small_b) {
+    /* (A: the ranks from n1 on, b1 <= b2) */
+    if (small_b)
+      for (uint32_t c = wid; c < ncand; c += NU_NW) {
+        const uint32_t r = readlane_u(cr, (int)c), s = readlane_u(cs, (int)c);
+        const int b = (int)readlane_u((uint32_t)cb, (int)c);
+        if (r >= n1 && r - n1 < A.n) continue;
         /* its bucket's elements are consecutive in the sorted set */
-        if (wid == (int)(c % NU_NW)) {
-          uint32_t before = 0u;
-          for (uint32_t i = lane; i - lane < B.n; i += WAVE)
-            before += (uint32_t)__popcll(__ballot(i < B.n && sel_bucket(key_x(L.ranked[min(i, B.n - 1u)]) - M) < b));
-          if (lane == 0) L.ckey[c] = L.ranked[min(before + (r - s), NU_SMALL - 1u)];
-        }
-        continue;
+        uint32_t before = 0u;
+        for (uint32_t i = lane; i - lane < B.n; i += WAVE)
+          before += (uint32_t)__popcll(__ballot(i < B.n && sel_bucket(key_x(L.ranked[min(i, B.n - 1u)]) - M) < b));
+        if (lane == 0) L.ckey[c] = L.ranked[min(before + (r - s), NU_SMALL - 1u)];
       }
-      const uint64_t key = nuc_select(in_a ? A : B, L, M, b, r - s);
+    for (uint32_t c = 0; c < ncand; c++) { /* (uniform; nuc_select takes L.ranked over) */
+      const uint32_t r = readlane_u(cr, (int)c), s = readlane_u(cs, (int)c);
+      const bool in_a = r >= n1 && r - n1 < A.n;
+      if (in_a ? small_a : small_b) continue;
+      const uint64_t key = nuc_select(in_a ? A : B, L, M, (int)readlane_u((uint32_t)cb, (int)c), r - s);
       if (tid == 0) L.ckey[c] = key;
     }
     __syncthreads();

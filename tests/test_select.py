@@ -326,3 +326,38 @@ def test_quantised_logits(gpu, oracle, dtype, N, V, k, step):
     u = oracle.uniform(25, V, N, k)
     for T in (1.0, 0.7):
         check(gpu, oracle, x, u, T, 0.97)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("V,k", [(8200, 8200), (24007, 24007), (24007, 5000), (100003, 100003)])
+def test_ids_only_small_temperatures_and_whole_rows(gpu, oracle, dtype, V, k):
+    """the wide nucleus kernels where the cut's bounds are hard to come by: T
+    from the smallest on (lse of some millions), top_p at and about 1 (cuts in the
+    last elements of any mass, or none), crowded and masked rows"""
+    rng = np.random.default_rng([V, k])
+    x = crowded_rows(rng, V, dtype)
+    u = oracle.uniform(31, k, len(x), k)
+    eps = np.float32(2.0 ** -24)
+    P = np.array([0.9, 1.0, 1 - eps, 1 + 2 * eps, 0.99999, 0.0, 0.5, 1.0, 1.0, 1.0, 1.0, 0.999], np.float32)
+    for T in (0.0, 0.1, 0.4, 1.0, 30.0):
+        check(gpu, oracle, x, u, T, P, want_probs=False)
+    ban = np.where(np.arange(12) % 2, 5, V - 1).astype(np.int32)
+    check(gpu, oracle, x, u, 0.0, 1.0, banned=ban, want_probs=False)
+    x = rows(rng, 24, V, dtype)  # (rounding decides whether the prefix passes 1)
+    check(gpu, oracle, x, oracle.uniform(32, k, 24, k), np.linspace(0.2, 2.0, 24).astype(np.float32), 1.0,
+          want_probs=False)
+
+
+def test_ids_only_winners_in_large_sets(gpu, oracle):
+    """the race won in a set of thousands of equal or nearly equal elements, by
+    rank: uniforms so small that those ranks win over all others"""
+    V = 40009
+    rng = np.random.default_rng(33)
+    x = np.stack([np.full(V, 2.0), np.round(rng.standard_normal(V) * 2), 1 + rng.random(V) * 1e-3,
+                  rng.standard_normal(V) * 1e-2]).astype(np.float32)
+    for at in (0, 1, 777, 20000, 39000):
+        u = oracle.uniform(34, at, 4, V)
+        u[:, at] = np.float32(2.0 ** -24)
+        u[:, at + 5] = np.float32(2.0 ** -23)
+        for T, P in ((1.0, 1.0), (0.5, 0.98), (1.0, 0.5)):
+            check(gpu, oracle, x, u, T, P, want_probs=False)
