@@ -22,9 +22,13 @@
  * candidates than k_nuc_race files, is sorted by k_nuc_final's workgroup.
  *
  * Bound: k_sel_hist's exponentials and each launch's latency.  [64, 151936]
- * bf16, N(0, 3) logits, top_p 0.9: 5.3 + 15.5 + 8.9 + 10.0 + 12.4 + 12.3 us (62 us
- * a call) against 175 us for the sorting kernels; N(0, 0.3) logits (93% of the
- * ranks kept) 149 against 182 us; one row 43 against 105 us. */
+ * bf16, N(0, 3) logits, top_p 0.9: 4.3 + 15.9 + 9.0 + 8.9 + 12.9 + 11.8 us (60 us
+ * a call) against 167 us for the sorting kernels, and at any T (T = 1e-5: 48
+ * against 241 us); top_p 1: 148 against 174 us; N(0, 0.3) logits (93% of the ranks
+ * kept) 140 against 174 us; one row 42 against 68 us, 70 against 75 us at top_p 1.
+ * Not everywhere: [64, 151936] of whole numbers at top_p 1 202 against 167 us, of
+ * one value 153 against 118 us (thousands of equal elements at the cut, searched
+ * by one workgroup a row). */
 #include <algorithm>
 
 #include "d3s_select.h"
@@ -41,7 +45,7 @@ struct NucRow {
   uint32_t b1, b2; /* the buckets the cut lies in; b1 > b2: the cut is k */
   uint32_t n1;     /* the elements before b1, and (q1) their sum of fix40(d3s_expf(x - m)) */
   uint32_t r1, r2; /* the ranks below r1 are kept, those from r2 on are not */
-  uint32_t open;   /* the cut is k unless it lies in b1 .. b2 (what follows adds nothing to the prefix) */
+  uint32_t open;   /* the cut is k unless it lies in b1 .. b2 (nothing, or nothing of any mass, follows) */
   uint64_t q1, qk; /* qk: the sum of all k (b1 > b2, or open) */
 };
 /* a share of the ranks: the least its best kept rank can score, and the ranks
@@ -74,7 +78,7 @@ constexpr int NU_T = 1024, NU_NW = NU_T / WAVE;
 constexpr uint32_t NU_SMALL = 512; /* gathered elements ranked by counting (a pass over all for each; past
                                       that a search narrows them, about three passes) */
 constexpr int NR_T = 512;          /* threads of a share's workgroup */
-constexpr uint32_t NU_TOP = 1024;  /* every share also looks at the first ranks */
+constexpr uint32_t NU_TOP = 512;   /* every share first looks at the first ranks */
 
 /* exclusive block scan of per-thread 64-bit values modulo 2^64; tot = total.
  * Ends with a barrier. */
@@ -92,6 +96,35 @@ __device__ __forceinline__ uint64_t nuc_scan(uint64_t v, uint64_t *sh, uint64_t 
   }
   __syncthreads();
   tot = t;
+  return base + inc - v;
+}
+
+/* the same for a count as well (shn: NU_NW words) */
+__device__ __forceinline__ uint64_t nuc_scan2(uint64_t v, uint32_t c, uint64_t *sh, uint32_t *shn, uint64_t &tot,
+                                              uint32_t &before, uint32_t &n) {
+  const int lane = lane_id(), wid = (int)threadIdx.x / WAVE;
+  const uint64_t inc = wave_scan_mod64(v);
+  const uint32_t cin = wave_scan_add_u32(c);
+  if (lane == WAVE - 1) {
+    sh[wid] = inc;
+    shn[wid] = cin;
+  }
+  __syncthreads();
+  uint64_t base = 0ull, t = 0ull;
+  uint32_t cb = 0u, ct = 0u;
+#pragma unroll 4
+  for (int w = 0; w < NU_NW; w++) {
+    const uint64_t x = sh[w];
+    const uint32_t y = shn[w];
+    base += w < wid ? x : 0ull;
+    cb += w < wid ? y : 0u;
+    t += x;
+    ct += y;
+  }
+  __syncthreads();
+  tot = t;
+  before = cb + cin - c;
+  n = ct;
   return base + inc - v;
 }
 
@@ -114,7 +147,11 @@ __device__ __forceinline__ bool nuc_races(float u) {
 /* bounds of the race's noise -d3s_logf(1 - u) for those u: from 2^-8 on the
  * hardware log (its error, at most 2^-23 |log2| + 2^-24, and 1 - u's rounding
  * are below 2^-14 of it there); below, u <= -log(1 - u) <= u + u^2, within
- * 2^-24 for 1 - u's rounding and the log's */
+ * 2^-24 for 1 - u's rounding and the log's, and at least 2^-24 (1 - u, as
+ * rounded, is at most 1 - 2^-24; the log's relative error there is 2^-24): without
+ * that a rank with u = 2^-24, one in 2^24, would count as able to win from
+ * anywhere, and the bucket of a row's far tail be gathered and searched */
+constexpr float NU_LEAST = 0x1p-24f * (1.0f - 0x1p-12f);
 __device__ __forceinline__ float nuc_noise_hi(float u) {
   const float a = -__builtin_amdgcn_logf(1.0f - u) * (LN2_F * (1.0f + 0x1p-12f));
   const float b = (__builtin_fmaf(u, u, u) + 0x1p-24f) * (1.0f + 0x1p-16f);
@@ -122,7 +159,7 @@ __device__ __forceinline__ float nuc_noise_hi(float u) {
 }
 __device__ __forceinline__ float nuc_noise_lo(float u) {
   const float a = -__builtin_amdgcn_logf(1.0f - u) * (LN2_F * (1.0f - 0x1p-12f));
-  const float b = (u - 0x1p-24f) * (1.0f - 0x1p-16f);
+  const float b = fmaxf((u - 0x1p-24f) * (1.0f - 0x1p-16f), NU_LEAST);
   return u < 0x1p-8f ? b : a;
 }
 
@@ -238,7 +275,7 @@ __global__ __launch_bounds__(NU_T) void k_nuc_bound(SampleArgs a, SelLayout F, N
   /* all k's sum is known when they end with a bucket, or in one of zero terms;
    * then only the buckets that can hold the cut are looked at */
   const bool known = start[bk + 1] == k || qv[2] == 0ull;
-  const bool whole = none && known, open = !none && known && b2 > bz;
+  const bool whole = none && known, open = !none && known && b2 == bk;
   /* R1 ranks are surely kept (rank 0 always is), none past R2 is */
   uint32_t R1 = k;
   const uint32_t R2 = none ? k : min(k, start[b2 + 1]);
@@ -257,7 +294,7 @@ __global__ __launch_bounds__(NU_T) void k_nuc_bound(SampleArgs a, SelLayout F, N
     r.lse = lse;
     r.state = NUC_LIVE;
     r.b1 = whole ? 1u : (uint32_t)b1;
-    r.b2 = whole ? 0u : (uint32_t)(open ? max(bz, b1) : b2);
+    r.b2 = whole ? 0u : (uint32_t)(open ? min(b2, max(bz, b1)) : b2);
     r.n1 = start[b1];
     r.r1 = R1;
     r.r2 = R2;
@@ -272,8 +309,8 @@ __global__ __launch_bounds__(NR_T) void k_nuc_race(SampleArgs a, NucLayout N) {
   __shared__ __align__(16) uint32_t start[SEL_NB + 4];
   __shared__ uint32_t nc;
   __shared__ float sb[NR_T / WAVE];
-  const int share = (int)blockIdx.x, row = (int)blockIdx.y, tid = (int)threadIdx.x, lane = lane_id();
-  const int wid = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int row = (int)blockIdx.y, tid = (int)threadIdx.x, lane = lane_id();
+  const uint32_t share = blockIdx.x, wid = (uint32_t)__builtin_amdgcn_readfirstlane(tid / WAVE);
   constexpr uint32_t NW = NR_T / WAVE;
   const NucRow *rec = N.row + row;
   const uint4 st = ((const uint4 *)(N.start + (size_t)row * SEL_NB))[tid];
@@ -286,33 +323,42 @@ __global__ __launch_bounds__(NR_T) void k_nuc_race(SampleArgs a, NucLayout N) {
   }
   __syncthreads();
   /* 64 ranks at a time, with the e of the block's first and last bucket, or of
-   * each rank's own where they lie further apart; the share's blocks to its
-   * waves in `unit`s, one round of bucket searches each */
-  const uint32_t nblk = (R2 + WAVE - 1) / WAVE, per = (nblk + gridDim.x - 1) / gridDim.x;
-  const uint32_t blk0 = min(nblk, share * per), blk1 = min(nblk, blk0 + per);
-  const uint32_t unit = min(64u, max(1u, (per + NW - 1) / NW));
+   * each rank's own where they lie further apart; the blocks to the shares' waves
+   * in `unit`s, one round of bucket searches each.  A share's units lie apart: it
+   * has surely kept ranks of its own among them, and a best score to measure the
+   * ranks near the cut by (a share of the last ranks alone filed too many). */
+  const uint32_t nblk = (R2 + WAVE - 1) / WAVE, shares = gridDim.x;
+  const uint32_t unit = min(64u, max(1u, (nblk + shares * NW - 1) / (shares * NW)));
   const float *urow = a.u + (size_t)row * a.k;
-  auto blocks = [&](auto &&fn) {
+  /* (the blocks some rank of which can score `reach`; with top_p near 1 or a low
+   * T most cannot, whatever their uniforms) */
+  auto blocks = [&](float reach, auto &&fn) {
 #pragma unroll 1
-    for (uint32_t k0 = blk0 + wid * unit; k0 < blk1; k0 += NW * unit) {
+    for (uint32_t k0 = (wid * shares + share) * unit; k0 < nblk; k0 += NW * shares * unit) {
       const uint32_t rb = min((k0 + (uint32_t)lane) * WAVE, R2 - 1), re = min(rb + WAVE - 1, R2 - 1);
       const int bf = nuc_bucket_of(start, rb), bl = nuc_bucket_of(start, re);
       const float hi = nuc_ehi(bf), lo = nuc_elo(bl);
-      const uint32_t kn = min(unit, blk1 - k0);
+      const uint32_t kn = min(unit, nblk - k0);
+      uint64_t todo = __ballot((uint32_t)lane < kn && hi * ((1.0f + 0x1p-10f) / NU_LEAST) >= reach);
 #pragma unroll 1
-      for (uint32_t j0 = 0; j0 < kn; j0 += 8) {
+      while (todo) {
         float u[8];
+        int at[8]; /* (uniform) */
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-          const uint32_t r = (k0 + j0 + j) * WAVE + lane;
-          u[j] = j0 + j < kn && r < R2 ? urow[r] : 2.0f;
+          at[j] = todo ? (int)__builtin_ctzll(todo) : -1;
+          todo &= todo - 1ull;
+          const uint32_t r = (k0 + (uint32_t)at[j]) * WAVE + lane;
+          u[j] = at[j] >= 0 && r < R2 ? urow[r] : 2.0f;
         }
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-          if (j0 + j >= kn) break; /* (uniform) */
-          const int l = (int)(j0 + j);
-          const uint32_t r = (k0 + j0 + j) * WAVE + lane;
+          if (at[j] < 0) break;
+          const int l = at[j];
+          const uint32_t r = (k0 + (uint32_t)l) * WAVE + lane;
           float h = readlane_f(hi, l), e = readlane_f(lo, l);
+          /* (noise is at least u - 2^-24) */
+          if (__ballot(u[j] * reach <= h * (1.0f + 0x1p-10f) + reach * 0x1p-23f) == 0ull) continue;
           if (readlane_u((uint32_t)bl, l) - readlane_u((uint32_t)bf, l) > 1u) {
             const int b = nuc_bucket_of(start, min(r, R2 - 1));
             h = nuc_ehi(b);
@@ -328,29 +374,32 @@ __global__ __launch_bounds__(NR_T) void k_nuc_race(SampleArgs a, NucLayout N) {
     const float lb = lo * __builtin_amdgcn_rcpf(nuc_noise_hi(u));
     if (r < R1 && nuc_races(u)) best = fmaxf(best, lb);
   };
+  auto all_waves = [&]() {
+    best = wave_max_f(best);
+    if (lane == 0) sb[wid] = best;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t w = 0; w < NW; w++) best = fmaxf(best, sb[w]);
+    __syncthreads();
+  };
   /* (the first ranks hold much of a peaked row's mass: a share whose own ranks
-   * are few, light or not surely kept still has a score to reach) */
-  if (blk0 > 0u) {
-    const uint32_t most = min(min(R1, NU_TOP), blk0 * WAVE);
-    float u[NU_TOP / NR_T];
+   * are few or light still has a score to reach) */
+  const uint32_t most = min(R1, NU_TOP);
+  float ut[NU_TOP / NR_T];
 #pragma unroll
-    for (uint32_t q = 0; q < NU_TOP / NR_T; q++) u[q] = tid + q * NR_T < most ? urow[tid + q * NR_T] : 2.0f;
+  for (uint32_t q = 0; q < NU_TOP / NR_T; q++) ut[q] = tid + q * NR_T < most ? urow[tid + q * NR_T] : 2.0f;
 #pragma unroll
-    for (uint32_t q = 0; q < NU_TOP / NR_T; q++)
-      if (tid + q * NR_T < most) least(tid + q * NR_T, u[q], 0.0f, nuc_elo(nuc_bucket_of(start, tid + q * NR_T)));
-  }
-  blocks(least);
-  best = wave_max_f(best);
-  if (lane == 0) sb[wid] = best;
-  __syncthreads();
-#pragma unroll
-  for (uint32_t w = 0; w < NW; w++) best = fmaxf(best, sb[w]);
+  for (uint32_t q = 0; q < NU_TOP / NR_T; q++)
+    if (tid + q * NR_T < most) least(tid + q * NR_T, ut[q], 0.0f, nuc_elo(nuc_bucket_of(start, tid + q * NR_T)));
+  all_waves();
+  blocks(best, least);
+  all_waves();
   best *= 1.0f - 0x1p-14f; /* (the reciprocal's error and the scores' own roundings) */
   NucShare *out = N.share + (size_t)row * BK_SMAX + share;
   const bool found = best > 0x1p-100f && best < 0x1p100f;
   if (found) {
     const float inv = __builtin_amdgcn_rcpf(best) * (1.0f + 0x1p-14f);
-    blocks([&](uint32_t r, float u, float hi, float) {
+    blocks(best, [&](uint32_t r, float u, float hi, float) {
       /* u <= -log(1 - u) + 2^-24, so this passes every rank whose score can reach best */
       if (r < R2 && nuc_races(u) && u <= hi * inv * (1.0f + 0x1p-14f) + 0x1p-23f) {
         const int b = nuc_bucket_of(start, r);
@@ -370,7 +419,7 @@ __global__ __launch_bounds__(NR_T) void k_nuc_race(SampleArgs a, NucLayout N) {
   __syncthreads();
   if (tid == 0) {
     out->best = found ? best : 0.0f;
-    out->n = blk0 < blk1 && !found ? NU_C + 1u : nc; /* (too many: the row is sorted) */
+    out->n = share * unit < nblk && !found ? NU_C + 1u : nc; /* (too many: the row is sorted) */
   }
 }
 
@@ -488,12 +537,16 @@ __global__ __launch_bounds__(SEL_T) void k_nuc_gather(SampleArgs a, SelLayout F,
   }
 }
 
-/* a gathered set */
+/* a gathered set.  Its keys are read 64 consecutive ones of a segment at a time,
+ * a wave each, the 64s numbered over the segments: lane s holds how many there
+ * are up to segment s, and how many keys s has, so a ballot finds the segment
+ * (a search by key in LDS took half of a pass) */
 struct NucSet {
   const uint64_t *keys;
   const uint32_t *base; /* LDS: the segments' places, BK_SMAX + 1 */
   int rstride;
   uint32_t n;
+  uint32_t upto, count; /* by lane */
   __device__ __forceinline__ uint64_t at(uint32_t i) const {
     int sg = 0;
 #pragma unroll
@@ -503,30 +556,41 @@ struct NucSet {
   /* fn(key) for each element, by the whole workgroup */
   template <class Fn>
   __device__ __forceinline__ void each(Fn &&fn) const {
+    const int lane = lane_id(), wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE);
+    const uint32_t all = readlane_u(upto, BK_SMAX - 1);
 #pragma unroll 1
-    for (uint32_t i0 = threadIdx.x; i0 < n; i0 += 4 * NU_T) {
-      uint64_t kv[4];
+    for (uint32_t c0 = wid; c0 < all; c0 += 8 * NU_NW) {
+      uint64_t kv[8];
+      uint32_t in = 0u;
 #pragma unroll
-      for (int q = 0; q < 4; q++) kv[q] = i0 + q * NU_T < n ? at(i0 + q * NU_T) : 0ull;
+      for (int q = 0; q < 8; q++) {
+        const uint32_t c = c0 + q * NU_NW;
+        const int sg = (int)__popcll(__ballot(lane < BK_SMAX && upto <= c)); /* (uniform; BK_SMAX past the last) */
+        const uint32_t first = sg ? readlane_u(upto, sg - 1) : 0u;
+        const uint32_t i = (c - first) * WAVE + lane;
+        const bool ok = c < all && i < readlane_u(count, sg);
+        in |= (ok ? 1u : 0u) << q;
+        kv[q] = ok ? keys[(size_t)sg * rstride + i] : 0ull;
+      }
 #pragma unroll
-      for (int q = 0; q < 4; q++)
-        if (i0 + q * NU_T < n) fn(kv[q]);
+      for (int q = 0; q < 8; q++)
+        if ((in >> q) & 1u) fn(kv[q]);
     }
   }
 };
 
-struct NucLds {
+struct __align__(16) NucLds {
   uint64_t list[NU_SMALL + 2], ranked[NU_SMALL];
   union {
     struct { /* a large set's counts and sums by 11 bits of what its keys span */
-      uint64_t ps[SEL_NB], ks[SEL_NB];
+      uint64_t ps[SEL_NB];
       uint32_t hist[SEL_NB];
     };
     struct { /* nuc_sort_row's places by wave and digit */
       uint32_t wcnt[NU_NW][NB], base[NB];
     };
   };
-  uint64_t sq[NU_NW], lo, hi, p, k;
+  uint64_t sq[NU_NW], lo, hi, p;
   uint32_t sh[NU_NW], n, above, count;
   int bin;
   uint32_t abase[BK_SMAX + 1], bbase[BK_SMAX + 1];
@@ -558,7 +622,13 @@ __device__ __forceinline__ void nuc_range(const NucSet &A, NucLds &L, uint64_t &
       hi = v > hi ? v : hi;
     }
   });
-  if (lo <= hi) {
+#pragma unroll
+  for (int sh = 1; sh < WAVE; sh <<= 1) {
+    const uint64_t l2 = (uint64_t)__shfl_xor((unsigned long long)lo, sh), h2 = (uint64_t)__shfl_xor((unsigned long long)hi, sh);
+    lo = l2 < lo ? l2 : lo;
+    hi = h2 > hi ? h2 : hi;
+  }
+  if (lane_id() == 0 && lo <= hi) { /* (an atomic a wave: 1024 on one word took 9 us) */
     atomicMin((unsigned long long *)&L.lo, (unsigned long long)lo);
     atomicMax((unsigned long long *)&L.hi, (unsigned long long)hi);
   }
@@ -567,14 +637,18 @@ __device__ __forceinline__ void nuc_range(const NucSet &A, NucLds &L, uint64_t &
   hi = L.hi;
 }
 
-/* the keys of a set for which in(key), at most NU_SMALL of them, ranked */
-template <class In>
-__device__ __forceinline__ uint32_t nuc_collect(const NucSet &A, NucLds &L, In &&in) {
+/* the keys of a set for which in(key), at most NU_SMALL of them, ranked;
+ * other(key) for the others */
+template <class In, class Other>
+__device__ __forceinline__ uint32_t nuc_collect(const NucSet &A, NucLds &L, In &&in, Other &&other) {
   __syncthreads();
   if (threadIdx.x == 0) L.n = 0u;
   __syncthreads();
   A.each([&](uint64_t key) {
-    if (in(key)) L.list[atomicAdd(&L.n, 1u)] = key;
+    if (in(key))
+      L.list[atomicAdd(&L.n, 1u)] = key;
+    else
+      other(key);
   });
   __syncthreads();
   const uint32_t n = L.n;
@@ -582,8 +656,8 @@ __device__ __forceinline__ uint32_t nuc_collect(const NucSet &A, NucLds &L, In &
   return n;
 }
 
-/* what a search for the cut has behind it: ranks, their sums of
- * fix40(d3s_expf(x - lse)) and of fix40(d3s_expf(x - m)) */
+/* what a search for the cut has behind it: ranks, and their sums of
+ * fix40(d3s_expf(x - lse)) (p) and of fix40(d3s_expf(x - m)) (k) */
 struct NucSum {
   uint32_t n;
   uint64_t p, k;
@@ -623,74 +697,93 @@ __device__ __forceinline__ bool nuc_cut_small(NucLds &L, uint32_t n, float M, fl
  * their counts and exact sums by 11 bits of it (the digits of a bucket's few
  * values lie apart, where the key's leading bytes are all the same); the first
  * digit whose last rank is dropped; and so on in that digit until its keys are
- * few (ranked) or equal. */
+ * few (ranked) or equal.  at.k only where the cut is found.  equal: the set's
+ * elements all are. */
 __device__ __forceinline__ bool nuc_cut_large(const NucSet &A, NucLds &L, float M, float lse, float top_p, uint32_t k,
-                                              NucSum &at) {
-  const int tid = (int)threadIdx.x;
+                                              NucSum &at, bool &equal) {
+  const int tid = (int)threadIdx.x, lane = lane_id();
   uint64_t lo, hi;
   nuc_range(A, L, lo, hi, [](uint64_t) { return true; }, [](uint64_t key) { return key >> 32; });
+  equal = lo == hi;
   uint32_t count = A.n;
 #pragma unroll 1
-  while (lo < hi) {
-    if (count <= NU_SMALL) {
-      const uint32_t n = nuc_collect(A, L, [&](uint64_t key) { return (key >> 32) >= lo && (key >> 32) <= hi; });
-      return nuc_cut_small(L, n, M, lse, top_p, k, at);
-    }
+  while (lo < hi && count > NU_SMALL) {
     const int shift = nuc_shift(hi - lo);
     static_assert(SEL_NB == 2 * NU_T, "a thread two digits");
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < 2; j++) {
       L.hist[tid + j * NU_T] = 0u;
-      L.ps[tid + j * NU_T] = L.ks[tid + j * NU_T] = 0ull;
+      L.ps[tid + j * NU_T] = 0ull;
     }
     if (tid == 0) L.bin = SEL_NB;
     __syncthreads();
     A.each([&](uint64_t key) {
-      const uint64_t o = key >> 32;
+      const uint32_t o = (uint32_t)(key >> 32);
       if (o >= lo && o <= hi) {
         const int d = (int)((hi - o) >> shift);
-        const float x = key_x(key);
-        const uint64_t f = d3s_fix40_exp(x - lse), e = d3s_fix40_exp(x - M);
-        atomicAdd(&L.hist[d], 1u);
-        if (f) atomicAdd((unsigned long long *)&L.ps[d], (unsigned long long)f);
-        if (e) atomicAdd((unsigned long long *)&L.ks[d], (unsigned long long)e);
+        const uint64_t f = d3s_fix40_exp(key_x(key) - lse);
+        auto add = [&](uint32_t c) {
+          atomicAdd(&L.hist[d], c);
+          if (f) atomicAdd((unsigned long long *)&L.ps[d], (unsigned long long)(f * c));
+        };
+        /* equal elements (rounded logits) by one of their lanes */
+        uint64_t left = __ballot(true);
+#pragma unroll 1
+        for (int t = 0; t < 4 && left; t++) {
+          const int l = (int)__builtin_ctzll(left);
+          const uint64_t same = __ballot(((left >> lane) & 1ull) && o == readlane_u(o, l));
+          if (__popcll(same) < 16) break;
+          if (lane == l) add((uint32_t)__popcll(same));
+          left &= ~same;
+        }
+        if ((left >> lane) & 1ull) add(1u);
       }
     });
     __syncthreads();
-    const uint32_t c0 = L.hist[2 * tid], c1 = L.hist[2 * tid + 1];
-    const uint64_t p0 = L.ps[2 * tid], p1 = L.ps[2 * tid + 1], k0 = L.ks[2 * tid], k1 = L.ks[2 * tid + 1];
-    uint32_t nt;
-    uint64_t pt, kt;
-    const uint32_t nb = at.n + block_excl_scan_u32<NU_NW>(c0 + c1, L.sh, nt);
-    const uint64_t pb = at.p + nuc_scan(p0 + p1, L.sq, pt), kb = at.k + nuc_scan(k0 + k1, L.sq, kt);
-    const bool past0 = c0 && nuc_past(nb + c0, pb + p0, k, top_p);
-    const bool past1 = c1 && nuc_past(nb + c0 + c1, pb + p0 + p1, k, top_p);
+    const uint2 c = ((const uint2 *)L.hist)[tid];
+    const ulonglong2 p = ((const ulonglong2 *)L.ps)[tid];
+    uint32_t nb, nt;
+    uint64_t pt;
+    const uint64_t pb = at.p + nuc_scan2(p.x + p.y, c.x + c.y, L.sq, L.sh, pt, nb, nt);
+    nb += at.n;
+    const bool past0 = c.x && nuc_past(nb + c.x, pb + p.x, k, top_p);
+    const bool past1 = c.y && nuc_past(nb + c.x + c.y, pb + p.x + p.y, k, top_p);
     const int b = wave_min_i32(past0 ? 2 * tid : past1 ? 2 * tid + 1 : SEL_NB);
-    if (lane_id() == 0 && b < SEL_NB) atomicMin(&L.bin, b);
+    if (lane == 0 && b < SEL_NB) atomicMin(&L.bin, b);
     __syncthreads();
     const int bin = L.bin;
     if (bin == SEL_NB) { /* no cut in the set */
       at.n += nt;
-      at.p += pt;
-      at.k += kt;
       return false;
     }
     if (tid == bin / 2) {
       const bool second = bin & 1;
-      L.n = nb + (second ? c0 : 0u);
-      L.p = pb + (second ? p0 : 0ull);
-      L.k = kb + (second ? k0 : 0ull);
-      L.count = second ? c1 : c0;
+      L.n = nb + (second ? c.x : 0u);
+      L.p = pb + (second ? p.x : 0ull);
+      L.count = second ? c.y : c.x;
     }
     __syncthreads();
     at.n = L.n;
     at.p = L.p;
-    at.k = L.k;
     count = L.count;
     hi -= (uint64_t)bin << shift;
     const uint64_t span = (1ull << shift) - 1ull;
     lo = hi - lo > span ? hi - span : lo;
+  }
+  /* the kept sum before the keys left, and those ranked, or all of them equal */
+  uint64_t above = 0ull, tot;
+  auto sum = [&](uint64_t key) { above += (key >> 32) > hi ? d3s_fix40_exp(key_x(key) - M) : 0ull; };
+  if (lo < hi) {
+    const uint32_t n = nuc_collect(A, L, [&](uint64_t key) { return (key >> 32) >= lo && (key >> 32) <= hi; }, sum);
+    (void)nuc_scan(above, L.sq, tot);
+    at.k += tot;
+    return nuc_cut_small(L, n, M, lse, top_p, k, at);
+  }
+  if (count < A.n) {
+    A.each(sum);
+    (void)nuc_scan(above, L.sq, tot);
+    at.k += tot;
   }
   /* `count` equal elements: the first rank j of them (not rank 0) past top_p, or rank k */
   const float x = d3s_from_ordkey((uint32_t)hi);
@@ -738,7 +831,7 @@ __device__ __forceinline__ uint64_t nuc_select(const NucSet &A, NucLds &L, float
     lo = top - lo > span ? top - span : lo;
     hi = top;
     if (count <= NU_SMALL) {
-      (void)nuc_collect(A, L, [&](uint64_t key) { return key >= lo && key <= hi && mine(key); });
+      (void)nuc_collect(A, L, [&](uint64_t key) { return key >= lo && key <= hi && mine(key); }, [](uint64_t) {});
       return L.ranked[need - 1u];
     }
   }
@@ -816,8 +909,12 @@ __device__ __forceinline__ void nuc_sort_row(const SampleArgs &a, int row, const
   generic_tail_opgraph<NU_T>(a, row, lse, rp.top_p, src);
 }
 
-template <bool BF16>
-__global__ __launch_bounds__(NU_T) void k_nuc_final(SampleArgs a, NucLayout N) {
+/* MINW: waves a SIMD that the registers must allow.  Two workgroups a CU (64
+ * registers, the rare paths spilling) when there are more rows than CUs, else
+ * one: [2048, 8193] 24.7 us a launch of 1024 rows against 33.4, but [64, 151936]
+ * 13.9 against 11.9 us. */
+template <bool BF16, int MINW>
+__global__ __launch_bounds__(NU_T, MINW) void k_nuc_final(SampleArgs a, NucLayout N) {
   __shared__ __align__(16) NucLds L;
   const int row = (int)blockIdx.x, tid = (int)threadIdx.x, lane = lane_id();
   const int wid = __builtin_amdgcn_readfirstlane(tid / WAVE);
@@ -867,23 +964,26 @@ __global__ __launch_bounds__(NU_T) void k_nuc_final(SampleArgs a, NucLayout N) {
       cu = a.u[(size_t)row * a.k + cr];
     }
     const uint64_t *keys = N.keys + (size_t)row * 2 * (size_t)N.vstride;
-    const NucSet A{keys, L.abase, N.rstride, L.abase[BK_SMAX]};
-    const NucSet B{keys + N.vstride, L.bbase, N.rstride, L.bbase[BK_SMAX]};
+    const NucSet A{keys, L.abase, N.rstride, L.abase[BK_SMAX], wave_scan_add_u32((sg.na + WAVE - 1) / WAVE), sg.na};
+    const NucSet B{keys + N.vstride, L.bbase, N.rstride, L.bbase[BK_SMAX], wave_scan_add_u32((sg.nb + WAVE - 1) / WAVE),
+                   sg.nb};
 
     /* ---- the cut and the kept sum */
     uint32_t cut = k;
     uint64_t kept = rec->qk;
     const bool small_a = A.n <= NU_SMALL;
+    bool whole_row = false; /* the row's elements are all equal: rank r is element r */
     if (b1 <= b2) {
       NucSum at{n1, P1, rec->q1};
-      bool hit;
+      bool hit, equal = false;
       if (small_a) {
         if ((uint32_t)tid < A.n) L.list[tid] = A.at((uint32_t)tid);
         __syncthreads();
         rank_by_count<NU_T>(L.list, A.n, (int)A.n, L.ranked);
         hit = nuc_cut_small(L, A.n, M, lse, top_p, k, at);
       } else {
-        hit = nuc_cut_large(A, L, M, lse, top_p, k, at);
+        hit = nuc_cut_large(A, L, M, lse, top_p, k, at, equal);
+        whole_row = equal && A.n == (uint32_t)a.vocab;
       }
       if (hit || !rec->open) {
         cut = min(k, at.n);
@@ -916,7 +1016,10 @@ __global__ __launch_bounds__(NU_T) void k_nuc_final(SampleArgs a, NucLayout N) {
       const uint32_t r = readlane_u(cr, (int)c), s = readlane_u(cs, (int)c);
       const bool in_a = r >= n1 && r - n1 < A.n;
       if (in_a ? small_a : small_b) continue;
-      const uint64_t key = nuc_select(in_a ? A : B, L, M, (int)readlane_u((uint32_t)cb, (int)c), r - s);
+      NucSet S = A;
+      if (!in_a) S = B;
+      const uint64_t key = whole_row ? composite_key(M, (int)r)
+                                     : nuc_select(S, L, M, (int)readlane_u((uint32_t)cb, (int)c), r - s);
       if (tid == 0) L.ckey[c] = key;
     }
     __syncthreads();
@@ -982,6 +1085,13 @@ bool launch_nucleus(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hi
   if (a.k <= generic_max_k()) {
     if (!rounds_pay(a, groups, 45.0, 6e-6, generic_us(a, dt))) return false;
   } else {
+    /* a few short bf16 rows, none of whose ranks top_p drops, at T = 1: two passes
+     * sort them, and the search near a prefix of 1 costs more ([1, 17000] 40 us
+     * against 44 us, [16, 20000] 47 against 52, [4, 32768] 50 against 53; at 50 000
+     * 51 us either way; fp32, four passes, [1, 20000] 58 against 49) */
+    if (dt == DT_BF16 && !a.temperature && a.temperature_scalar == 1.0f && !a.top_p && a.top_p_scalar >= 1.0f &&
+        a.vocab <= 40000 && a.n_rows <= 32)
+      return false;
     const int64_t sorted = std::max<int64_t>(1, (int64_t)(ws_bytes / bigk_row_bytes(a)));
     const double sort_us = (double)((a.n_rows + sorted - 1) / sorted) * (30.0 + 4.5e-4 * a.vocab);
     if (!rounds_pay(a, groups, 45.0, -3e-6, sort_us)) return false; /* (4 against 7 ps an element) */
@@ -1005,13 +1115,14 @@ bool launch_nucleus(const SampleArgs &a, Dtype dt, void *ws, size_t ws_bytes, hi
     const dim3 grid((unsigned)F.nseg, (unsigned)n);
     hipLaunchKernelGGL(k_nuc_bound, dim3((unsigned)n), dim3(NU_T), 0, s, c, F, N);
     hipLaunchKernelGGL(k_nuc_race, grid, dim3(NR_T), 0, s, c, N);
-    if (dt == DT_F32) {
+    const bool f32 = dt == DT_F32, two = n > 256;
+    if (f32)
       hipLaunchKernelGGL(k_nuc_gather<false>, grid, dim3(SEL_T), 0, s, c, F, N);
-      hipLaunchKernelGGL(k_nuc_final<false>, dim3((unsigned)n), dim3(NU_T), 0, s, c, N);
-    } else {
+    else
       hipLaunchKernelGGL(k_nuc_gather<true>, grid, dim3(SEL_T), 0, s, c, F, N);
-      hipLaunchKernelGGL(k_nuc_final<true>, dim3((unsigned)n), dim3(NU_T), 0, s, c, N);
-    }
+    const auto last = f32 ? (two ? k_nuc_final<false, 8> : k_nuc_final<false, 4>)
+                          : (two ? k_nuc_final<true, 8> : k_nuc_final<true, 4>);
+    hipLaunchKernelGGL(last, dim3((unsigned)n), dim3(NU_T), 0, s, c, N);
   }
   return true;
 }

@@ -121,6 +121,24 @@ __global__ __launch_bounds__(SEL_T) void k_sel_hist(SampleArgs a, SelLayout L) {
     constexpr int EPC = BF16 ? 8 : 4;
     float x[EPC];
     sel_scale(v, T, y, te, x);
+    if (SUMS) { /* nearly equal rows: the lanes' equal elements added by one of them */
+      const float v0 = readlane_f(v[0], 0);
+      if (__popcll(__ballot(v[0] == v0)) > WAVE / 2) {
+        const float z0 = readlane_f(x[0], 0) - M;
+        const int b0 = sel_bucket(z0);
+        uint32_t same = 0u;
+#pragma unroll
+        for (int e = 0; e < EPC; e++) {
+          const bool eq = ((ok >> e) & 1u) && d3s_f2u(x[e]) == d3s_f2u(readlane_f(x[0], 0));
+          same += (uint32_t)__popcll(__ballot(eq));
+          ok &= ~((eq ? 1u : 0u) << e);
+        }
+        if (lane_id() == 0 && same && b0 < SEL_NB - 1) {
+          atomicAdd(&cnt[b0], same);
+          atomicAdd((unsigned long long *)&bsum[b0], (unsigned long long)(d3s_fix40_exp(z0) * same));
+        }
+      }
+    }
 #pragma unroll
     for (int e = 0; e < EPC; e++) {
       const float z = x[e] - M;

@@ -343,9 +343,22 @@ def test_ids_only_small_temperatures_and_whole_rows(gpu, oracle, dtype, V, k):
         check(gpu, oracle, x, u, T, P, want_probs=False)
     ban = np.where(np.arange(12) % 2, 5, V - 1).astype(np.int32)
     check(gpu, oracle, x, u, 0.0, 1.0, banned=ban, want_probs=False)
+    check(gpu, oracle, x[:5], u[:5], 1.0, 1.0, want_probs=False)  # (short bf16 rows: sorted)
+    check(gpu, oracle, x[5:], u[5:], 1.0, 1.5, want_probs=False)
     x = rows(rng, 24, V, dtype)  # (rounding decides whether the prefix passes 1)
     check(gpu, oracle, x, oracle.uniform(32, k, 24, k), np.linspace(0.2, 2.0, 24).astype(np.float32), 1.0,
           want_probs=False)
+
+
+def test_ids_only_many_rows(gpu, oracle):
+    """more rows than CUs (k_nuc_final's other form)"""
+    rng = np.random.default_rng(35)
+    N, V = 300, 8200
+    x = rows(rng, N, V, "bf16", 1.0)
+    x[::3] = W.f32_to_bf16_bits(np.round(rng.standard_normal((100, V)) * 2).astype(np.float32))
+    u = oracle.uniform(36, 1, N, V)
+    P = np.where(np.arange(N) % 2, 1.0, 0.9).astype(np.float32)
+    check(gpu, oracle, x, u, 0.7, P, want_probs=False)
 
 
 def test_ids_only_winners_in_large_sets(gpu, oracle):
