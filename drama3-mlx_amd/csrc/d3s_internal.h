@@ -106,7 +106,7 @@ void *stream_workspace(hipStream_t s, size_t bytes);
 void *stream_workspace_optional(hipStream_t s, size_t bytes, size_t *got);
 /* Waits for the stream, then frees its block and the blocks it outgrew. */
 int release_stream_workspace(hipStream_t s);
-/* Launch the head's gemv: up to two rows by k_linear, more by launch_linear_rows. */
+/* Launch the head's gemv: few rows or few logits by k_linear, else launch_linear_rows. */
 void launch_linear(const LinearArgs &la, hipStream_t s);
 /* Launch the gemv of several rows on the matrix cores (the same bits). */
 void launch_linear_rows(const LinearArgs &la, hipStream_t s);

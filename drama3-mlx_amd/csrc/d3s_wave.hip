@@ -1320,9 +1320,18 @@ void launch_ras_select(const RasArgs &r, const int32_t *first, const int32_t *re
 }
 
 void launch_linear(const LinearArgs &la, hipStream_t s) {
-  /* two rows are still faster one after the other (6.3 us against 7.6 us on
-   * [2, 2048] x [4097, 2048]; three rows 9.3 against 7.6 us) */
-  if (la.n_rows > 2) {
+  /* Several rows go to the matrix cores where there are logits enough: the rows
+   * kernel's workgroup takes its whole K one 128-element block after the other (2.2
+   * us a 1024 elements), k_linear a logit a half-wave with 16 blocks in flight
+   * (0.5 us), so few logits are done sooner there.  k_linear against the rows
+   * kernel: [3, 2048] x [1000, 2048] 3.9 and 6.8 us, [8, 4096] x [64, 4096] 4.2 and
+   * 11.1, [16, 1024] x [1000, 1024] 5.4 and 4.5, [3, 2048] x [4097, 2048] 9.3 and
+   * 7.1, two rows of that 6.3 and 7.6.  Three rows whose weights fit the L2s are read as fast
+   * again for each row as the tiles of a second round of workgroups: [3, 2048] x
+   * [8192, 2048] 13.0 and 14.6 us, [3, 4096] x [8192, 4096] 37.9 and 26.4. */
+  const int64_t logits = (int64_t)la.n_rows * la.V;
+  const bool three = la.n_rows == 3 && la.V > 4100 && la.K >= 512 && (int64_t)la.V * la.K <= 20000000;
+  if (la.n_rows > 2 && logits > 10240 && !three) {
     launch_linear_rows(la, s);
     return;
   }
