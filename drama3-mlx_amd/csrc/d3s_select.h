@@ -15,7 +15,7 @@ constexpr int SEL_WGS = 512;         /* workgroups a launch aims at: two per CU 
 constexpr int SEL_NB = 2048;         /* buckets below a row's max */
 constexpr float SEL_SCALE = 64.0f;   /* buckets per unit of x: 32 units, where the terms of the
                                         exact sum end (e^-28 < 2^-40) */
-constexpr float SEL_NEAR = 8.0f;     /* the selection's buckets: this, plus the distance, by its */
+constexpr float SEL_NEAR = 2.0f;     /* the selection's buckets: this, plus the distance, by its */
 constexpr int SEL_OCT_LOG2 = 8;      /* exponent and 8 mantissa bits: 8 octaves of 256 */
 constexpr int SEL_G = 32;            /* buckets a group */
 constexpr int SEL_NG = SEL_NB / SEL_G;
@@ -260,9 +260,9 @@ __device__ __forceinline__ float sel_logit_bound(float M, float T, int b) {
 /* The selection's buckets, of z times s = sel_rank_scale(T): what they divide
  * is a row's logits, since the k-th of a model's logits lies at some 8 to 15
  * units of L below the first at any T (x = L / T: 0.5 to 1.5 million at the
- * smallest T, where buckets of x held nearly all of a row in the last).  1/32
- * wide in the first 8 units, 1/16 to 24, and so on to 2040 units: rows of other
- * scales keep a relative width of 1/256.  (Equal widths and then 32 an octave,
+ * smallest T, where buckets of x held nearly all of a row in the last).  1/128
+ * wide in the first 2 units, 1/32 from 6 to 14, and so on to 510 units: rows of
+ * other scales keep a relative width of 1/256.  (Equal widths and then 32 an octave,
  * four instructions an element more: 540 us against 490 us at [256, 700001].) */
 __device__ __forceinline__ float sel_rank_scale(float T) { return fminf(T, 1.0f); }
 

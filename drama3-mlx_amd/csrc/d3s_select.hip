@@ -143,15 +143,18 @@ __global__ __launch_bounds__(SEL_T) void k_sel_hist(SampleArgs a, SelLayout L) {
     for (int e = 0; e < EPC; e++) {
       const float z = x[e] - M;
       const int b = SUMS ? sel_bucket(z) : sel_rank_bucket(z, s);
-      const bool in = (ok >> e) & 1u;
-      /* (the last bucket, where a row's masked or far elements all lie, has no
-       * terms, and its count, kept as 0, is what the others leave of the row: no
-       * atomics on one word) */
-      if (in && b < SEL_NB - 1) {
-        atomicAdd(&cnt[b], 1u);
-        if (SUMS) atomicAdd((unsigned long long *)&bsum[b], (unsigned long long)d3s_fix40_exp(z));
+      /* (the last bucket, where a row's masked or far elements all lie, and those
+       * outside the row, has no terms, and its count, kept as 0, is what the others
+       * leave of the row: no atomics on one word) */
+      if (SUMS) {
+        if (((ok >> e) & 1u) && b < SEL_NB - 1) {
+          atomicAdd(&cnt[b], 1u);
+          atomicAdd((unsigned long long *)&bsum[b], (unsigned long long)d3s_fix40_exp(z));
+        }
+      } else {
+        if (b < SEL_NB - 1) atomicAdd(&cnt[b], 1u);
+        acc += d3s_fix40_exp(z);
       }
-      if (!SUMS && in) acc += d3s_fix40_exp(z);
     }
   });
   const size_t at = (size_t)row * L.nseg + seg;
@@ -261,8 +264,10 @@ __global__ __launch_bounds__(SEL_T) void k_sel_gather(SampleArgs a, SelLayout L,
         at_b + 1 < SEL_G ? readlane_u(fin, min(at_b + 1, SEL_G - 1)) : readlane_u(gin, min(tg + 1, WAVE - 1));
     const float xc = Lc * y; /* (a little below Lc / T) */
     const int reach = sel_rank_bucket(fminf(xc - fabsf(xc) * 0x1p-20f - M, 0.0f), s);
-    /* (uniform; the last bucket's elements are not in the counts) */
-    if (__builtin_expect(next > (uint32_t)SEL_CAP || reach > tb + 1 || tb + 2 >= SEL_NB, 0)) {
+    /* (the last bucket's elements are not in the counts; a scalar branch lets the
+     * rare path lie out of line) */
+    const int rare = next > (uint32_t)SEL_CAP || reach > tb + 1 || tb + 2 >= SEL_NB ? 1 : 0;
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(rare) != 0, 0)) {
       crowd = tb == SEL_NB - 1 || readlane_u(fin, at_b) > (uint32_t)SEL_CAP;
       Lc = sel_rank_least(M, T, y, s, crowd ? tb - 1 : tb);
     }
@@ -667,7 +672,7 @@ __global__ __launch_bounds__(GBLOCK) void k_sel_sort(SampleArgs a, SelLayout L, 
   const uint32_t segn = lane < L.nseg ? sg0[lane].count : 0u;
   const uint64_t segs = lane < L.nseg ? sg0[lane].sum : 0ull;
   const uint32_t crowd = sg0[0].crowd;
-  const float least = sg0[0].least;
+  const float least = NQ > 1 ? sg0[0].least : 0.0f;
   float u[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; q++) {
@@ -684,13 +689,21 @@ __global__ __launch_bounds__(GBLOCK) void k_sel_sort(SampleArgs a, SelLayout L, 
   }
   const uint32_t inc = wave_scan_add_u32(segn);
   const uint32_t n = readlane_u(inc, WAVE - 1);
-  if (__builtin_expect(crowd != 0u, 0)) sel_crowd<BF16>(a, row, rp, M, (int)crowd - 1, n, sorted, bk, start, sh);
+  if (__builtin_expect(__builtin_amdgcn_readfirstlane((int)crowd) != 0, 0)) sel_crowd<BF16>(a, row, rp, M, (int)crowd - 1, n, sorted, bk, start, sh);
   const float lse = M + d3s_logf(d3s_fixsum_to_f32(wave_sum_mod64(segs)));
-  /* the gathered keys' buckets: SEL_NB equal parts of about what they span (any
-   * factor ranks them) */
-  const float span = M - least * y;
-  const float per = span > 0.0f ? fminf((float)SEL_NB * __builtin_amdgcn_rcpf(span), 0x1p100f) : 0.0f;
-  auto place = [&](float x) { return (int)fminf((M - x) * per, (float)(SEL_NB - 1)); };
+  /* their buckets: the selection's, or for many keys SEL_NB equal parts of about
+   * what they span (any factor ranks them; for few the load and the reciprocal
+   * cost more than they save: 8.9 against 9.4 us at k = 30, but [1024, 20000], k =
+   * 4096: 165 against 141 us a call) */
+  float per = 0.0f;
+  if (NQ > 1) {
+    const float span = M - least * y;
+    per = span > 0.0f ? fminf((float)SEL_NB * __builtin_amdgcn_rcpf(span), 0x1p100f) : 0.0f;
+  }
+  const float s = sel_rank_scale(T);
+  auto place = [&](float x) {
+    return NQ > 1 ? (int)fminf((M - x) * per, (float)(SEL_NB - 1)) : sel_rank_bucket(x - M, s);
+  };
   next[tid] = 0u;
   next[tid + GBLOCK] = 0u;
   if (tid == 0) many = 0u;
@@ -724,7 +737,7 @@ __global__ __launch_bounds__(GBLOCK) void k_sel_sort(SampleArgs a, SelLayout L, 
   if (max(c.x, c.y) * ((n + GBLOCK - 1) / GBLOCK) > SEL_PAIRS) many = 1u;
   uint32_t all;
   const uint32_t before = block_excl_scan_u32<GNW>(c.x + c.y, sh, all);
-  if (__builtin_expect(many != 0u, 0)) { /* (uniform: the scan's barriers) */
+  if (__builtin_expect(__builtin_amdgcn_readfirstlane((int)many) != 0, 0)) { /* (the scan's barriers stand between) */
     sel_radix<NK>(kv, n, bk, tab, sh);
     for (int i = tid; i < min((int)n, a.k); i += GBLOCK) sorted[i] = bk[i];
   } else {
