@@ -18,8 +18,9 @@
  *     ranks' elements (by sorting a small gathered set, by counting 11 bits of
  *     what its keys span in a large one: crowded ties, top_p near 1), their exact
  *     scores and the id.
- * A row whose kept ranks have no positive score (u = 0 throughout), or more
- * candidates than k_nuc_race files, is sorted by k_nuc_final's workgroup.
+ * A row no rank of which can score (u = 0 throughout) is its first rank's.  One
+ * whose kept ranks alone have no positive score, or with more candidates than
+ * k_nuc_race files, is sorted by k_nuc_final's workgroup (1.4 ms at V = 151 936).
  *
  * Bound: k_sel_hist's exponentials and each launch's latency.  [64, 151936]
  * bf16, N(0, 3) logits, top_p 0.9: 4.3 + 15.9 + 9.0 + 8.9 + 12.9 + 11.8 us (60 us
@@ -838,6 +839,45 @@ __device__ __forceinline__ uint64_t nuc_select(const NucSet &A, NucLds &L, float
   return hi;
 }
 
+/* whether no rank of the row scores (1 - u, as rounded, is 1, negative or NaN for
+ * all: every score counts as -1); by the whole workgroup */
+__device__ __forceinline__ bool nuc_none_scores(const SampleArgs &a, int row) {
+  const float *u = a.u + (size_t)row * a.k;
+  int none = 1;
+#pragma unroll 8
+  for (int r = (int)threadIdx.x; r < a.k; r += NU_T) {
+    const float w = 1.0f - u[r];
+    none &= w == 1.0f || !(w >= 0.0f) ? 1 : 0;
+  }
+  return __syncthreads_and(none) != 0;
+}
+
+/* the row's first rank: its greatest composite key */
+template <bool BF16>
+__device__ __forceinline__ void nuc_first_rank(const SampleArgs &a, int row, NucLds &L, const RowP &rp) {
+  const char *rowp = (const char *)a.logits + (size_t)row * (size_t)a.row_stride * (BF16 ? 2 : 4);
+  const float y = 1.0f / rp.T;
+  uint64_t top = 0ull;
+#pragma unroll 8
+  for (int i = (int)threadIdx.x; i < a.vocab; i += NU_T) {
+    const uint64_t key =
+        composite_key(scale_logit(load_logit<BF16>(rowp, i, rp.banned), rp.T, y, rp.T < __builtin_inff()), i);
+    top = key > top ? key : top;
+  }
+#pragma unroll
+  for (int sh = 1; sh < WAVE; sh <<= 1) {
+    const uint64_t o = (uint64_t)__shfl_xor((unsigned long long)top, sh);
+    top = o > top ? o : top;
+  }
+  if (lane_id() == 0) L.sq[threadIdx.x / WAVE] = top;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    top = L.sq[0];
+    for (int w = 1; w < NU_NW; w++) top = L.sq[w] > top ? L.sq[w] : top;
+    a.ids[row] = key_idx(top);
+  }
+}
+
 /* the row sorted by one workgroup (a stable LSD radix sort by ordkey(x)
  * descending, as k_bk_pass's tiles do it), and the op graph's tail over it: the
  * rare rows nothing else settles */
@@ -1046,6 +1086,10 @@ __global__ __launch_bounds__(NU_T, MINW) void k_nuc_final(SampleArgs a, NucLayou
   }
 sort:
   __syncthreads();
+  if (nuc_none_scores(a, row)) {
+    nuc_first_rank<BF16>(a, row, L, rp);
+    return;
+  }
   nuc_sort_row<BF16>(a, row, N, L, lse, rp);
 }
 

@@ -374,3 +374,20 @@ def test_ids_only_winners_in_large_sets(gpu, oracle):
         u[:, at + 5] = np.float32(2.0 ** -23)
         for T, P in ((1.0, 1.0), (0.5, 0.98), (1.0, 0.5)):
             check(gpu, oracle, x, u, T, P, want_probs=False)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_ids_only_where_no_rank_scores(gpu, oracle, dtype):
+    """uniforms for which every score counts as -1: the first rank; and one rank
+    that does score, kept or dropped"""
+    rng = np.random.default_rng(37)
+    x = crowded_rows(rng, 20011, dtype)
+    u = np.zeros((12, 20011), np.float32)
+    u[1] = 1.5
+    u[2] = 2.0 ** -26
+    u[3, ::2] = np.nan
+    u[7, 19999] = 0.25
+    u[8, 3] = 1.0
+    u[9, 0] = 0.5
+    for T, P in ((1.0, 0.9), (0.0, 1.0), (0.7, 0.3)):
+        check(gpu, oracle, x, u, T, P, want_probs=False)
