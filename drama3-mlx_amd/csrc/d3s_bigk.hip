@@ -7,8 +7,8 @@
  * up to 16 segments of whole 1024-key tiles, so a launch of few rows still
  * spreads over the CUs; six launches, 1024 threads a workgroup.  With k at most
  * V / 2 the selecting kernels (d3s_select.hip) come first and leave only the
- * elements that can rank below k ([16, 151936] fp32, k = 8000: 71 us against
- * 417 us by the streaming kernel; [1024, 20000] bf16, k = 6000: 173 us against
+ * elements that can rank below k ([16, 151936] fp32, k = 8000: 72 us against
+ * 420 us by the streaming kernel; [1024, 20000] bf16, k = 6000: 244 us against
  * 400 us); otherwise
  *  k_bk_keys (a workgroup per segment): x = L / T, classification and the
  *     segment's max; the composite keys (ordkey(x), ~index) written to the

@@ -26,7 +26,7 @@
  * bf16, N(0, 3) logits, top_p 0.9: 4.3 + 15.9 + 9.0 + 8.9 + 12.9 + 11.8 us (60 us
  * a call) against 167 us for the sorting kernels, and at any T (T = 1e-5: 48
  * against 241 us); top_p 1: 148 against 174 us; N(0, 0.3) logits (93% of the ranks
- * kept) 140 against 174 us; one row 42 against 68 us, 70 against 75 us at top_p 1.
+ * kept) 140 against 174 us; one row 42 against 68 us, 72 against 75 us at top_p 1.
  * Not everywhere: [64, 151936] of whole numbers at top_p 1 202 against 167 us, of
  * one value 153 against 118 us (thousands of equal elements at the cut, searched
  * by one workgroup a row). */

@@ -26,9 +26,9 @@
  * result is the oracle's bits.
  *
  * Bound: latency (four launches; k_sel_sort is one workgroup's chain).
- * [32, 151936] bf16, k = 1000: 3.6 + 10.5 + 8.1 + 13.1 us against 438 us for
- * k_generic, one workgroup a row; [1, 8193], k = 65: 20.7 us against 31.3 us;
- * [2048, 32768], k = 4096: 373 us against 776 us. */
+ * [32, 151936] bf16, k = 1000: 3.9 + 8.2 + 8.4 + 13.6 us against 436 us for
+ * k_generic, one workgroup a row (T = 1e-5: 33 us a call against 418); [1, 8193], k
+ * = 65: 19.6 us against 35.5 us; [2048, 32768], k = 4096: 384 us against 781 us. */
 #include <atomic>
 
 #include "d3s_rowcore.h"

@@ -106,7 +106,10 @@ extern "C" {
  * A row whose x are all -inf gets ids = 0 (the reference kernel's answer).
  * The result is identical for every flag combination.
  * The workspace comes from the block the library keeps for `stream` (see
- * Workspace above); d3s_sample_ws takes the caller's.
+ * Workspace above); d3s_sample_ws takes the caller's.  While the stream is being
+ * captured, calls that require none (64 < k <= 16384 on rows longer than 8192) take
+ * none, since a graph may outlive the block, and run on one workgroup a row: to
+ * capture the faster kernels, give a workspace.
  * Replaces: sample_with_noise (src/sampling.c:194-203, declared src/model.h:175-176). */
 int d3s_sample(const void *logits, int dtype, int64_t n_rows, int64_t vocab, int64_t row_stride,
                const float *u, int k, const float *temperature, const float *top_p,
@@ -118,18 +121,23 @@ int d3s_sample(const void *logits, int dtype, int64_t n_rows, int64_t vocab, int
  * the call's route keeps no state in device memory), or a negative status for
  * arguments d3s_sample rejects.  The need depends on dtype, n_rows, vocab, k
  * and flags (and on D3_NO_FUSED_SAMPLER only through the route, not the size).
- * For 64 < k <= 16384 on rows longer than 8192 it is the size with which the
- * rows are spread over the chip; a smaller workspace, or none, is accepted
- * there and gives the same results more slowly (for larger k: one that holds
- * a row's sort keys).
+ * For k > 64 on rows longer than 8192 this is the size with which the rows are
+ * spread over the chip, and not all of it is required: none of it for k <= 16384
+ * (a smaller workspace, or none, gives the same results more slowly), and for
+ * larger k the sort keys of every row (16 bytes an element and 97 KiB a row, up
+ * to 256 MiB in all).  A smaller workspace than this is used where the rows it
+ * holds at a time make few enough rounds of launches (about 22 us each for k <=
+ * 4096, 45 to 55 us beyond) to beat one launch of the streaming kernel, else it is
+ * left alone.
  * Replaces the one-time set-up of sample_kernel_call (src/sampling.c:142-157). */
 int64_t d3s_sample_workspace_bytes(int dtype, int64_t n_rows, int64_t vocab, int k, unsigned flags);
 
 /* d3s_sample with the workspace given: never allocates, so it may be captured
  * in a HIP graph.  workspace: device memory of workspace_bytes (256-byte
  * aligned, cleared once by d3s_workspace_init; it may be NULL when
- * d3s_sample_workspace_bytes is 0).  A workspace smaller than the call needs
- * returns D3S_ERR_WORKSPACE before anything is launched.  Calls that share a
+ * d3s_sample_workspace_bytes is 0, or k <= 16384 on rows longer than 8192).  A
+ * workspace smaller than the call requires returns D3S_ERR_WORKSPACE before
+ * anything is launched.  Calls that share a
  * workspace must run one after another (one stream).  Same results as
  * d3s_sample. */
 int d3s_sample_ws(const void *logits, int dtype, int64_t n_rows, int64_t vocab, int64_t row_stride,
@@ -162,7 +170,10 @@ int d3s_stream_workspace_release(void *stream);
  * in the library's static device memory, held until the process ends.  Every
  * call the segmented kernel takes fits (it takes at most 4096 segments per
  * launch: 256 KiB of counters and at most 2.1 MiB of records); a call that
- * would not returns D3S_ERR_SCRATCH.
+ * would not returns D3S_ERR_SCRATCH.  For k > 64 on rows longer than 8192 the
+ * selecting, wide nucleus and sorting kernels keep as many rows' state there as
+ * fit, where that is worth it (k > 16384 on rows longer than 239 296 returns
+ * D3S_ERR_SCRATCH).
  * All calls on one GPU share that block: calls that overlap on one GPU
  * (several streams or threads at once) race and must not be issued. */
 int d3s_sample_noalloc(const void *logits, int dtype, int64_t n_rows, int64_t vocab, int64_t row_stride,
@@ -205,7 +216,9 @@ typedef struct {
  * (the retry's indices go to retry_idx, else to code0, else to the
  * workspace).  The workspace, when the draws' routes or the retry's indices
  * need one, comes from the block the library keeps for `stream` (see
- * Workspace above; D3S_ERR_NOMEM if it cannot be allocated).
+ * Workspace above; D3S_ERR_NOMEM if it cannot be allocated).  It holds what the
+ * draws require and no more: with 64 < k <= 16384 on rows longer than 8192 they run
+ * on one workgroup a row, where d3s_sample spreads rows over the chip.
  * Replaces: the two sample_with_noise calls, candidate_token and the repeat test of
  * tower_decode_step (src/tower.c:420-433). */
 int d3s_sample_ras(const void *logits, int dtype, int64_t n_rows, int64_t vocab, int64_t row_stride,
@@ -256,7 +269,9 @@ int d3s_linear_bf16(const uint16_t *x, const uint16_t *w, int64_t n_rows, int64_
  * instead of two, about 2 us slower on [1, 2048] x [4097, 2048]); other
  * calls take the two launches.  A workspace, when the call needs one, comes
  * from the block the library keeps for `stream` (see Workspace above;
- * D3S_ERR_NOMEM if it cannot be allocated).
+ * D3S_ERR_NOMEM if it cannot be allocated).  It holds what the sample requires
+ * and no more: with 64 < k <= 16384 and V > 8192 the sample runs on one workgroup a
+ * row (d3s_linear_bf16 and d3s_sample on its logits spread it over the chip).
  * Replaces: m_linear through gemv_row (src/mlxu.c:454-496) followed by
  * sample_with_noise on its logits: the backbone head (src/backbone.c:1213-1215)
  * and the tower's codebook heads (src/tower.c:228-232,:264,:440-443). */
